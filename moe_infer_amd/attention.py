@@ -23,8 +23,6 @@ Reference operators these stand for (fbundle/moe_infer):
 """
 from __future__ import annotations
 
-import ctypes as C
-
 import torch
 
 from . import _lib
@@ -34,15 +32,25 @@ KV_KBLOCK = 32
 KV_VBLOCK = 8
 
 
-def _stream() -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+# A decode step is about 10 us of GPU work, so what the host spends per call
+# decides how fast short calls go.  Measured per call: torch.cuda.current_stream()
+# 2.9 us against 0.1 us for the raw handle; a tensor's five checks one by one
+# 0.55 us against 0.3 us as one expression; a c_void_p object per pointer 0.15 us
+# (ctypes takes the address as an int).
+def _stream() -> int:
+    """The current HIP stream of the current device."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
-def _ptr(t: torch.Tensor | None) -> C.c_void_p | None:
-    return None if t is None else C.c_void_p(t.data_ptr())
+def _ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
 
 
 def _check_tensor(name: str, t: torch.Tensor, numel: int, dtype=torch.float16) -> None:
+    if (isinstance(t, torch.Tensor) and t.dtype is dtype and t.is_cuda and t.is_contiguous()
+            and t.numel() == numel and not t.data_ptr() & 15):
+        return
+    # which of them failed
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
     if t.dtype != dtype:

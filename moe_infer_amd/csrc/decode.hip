@@ -119,24 +119,28 @@ __device__ __forceinline__ f16x8 load16(const _Float16* p) {
 // kernel.  cos / sin of the rotation angles pos * inv_freq[i] are computed on
 // the host (the position is a host value), in f32 like the reference:
 // cs[i] = cos, cs[rot_half + i] = sin, i < rot_half.
-struct ProjArgs {
+struct ProjInput {
   const float* q_proj;  // [H][2*D]: query then gate of each head
   const float* k;       // [G][D]
   const float* v;       // [G][D]
   const uint16_t* q_w;  // bf16 [D]
   const uint16_t* k_w;  // bf16 [D]
-  int rot_half;          // host side: selects the Proj<rot_half / 32> kernel
   float eps;
+};
+struct ProjArgs : ProjInput {
+  int rot_half;  // host side: selects the Proj<rot_half / 32> kernel
   float cs[MI_ROPE_MAX_DIM];
 };
 struct NoProj {
   static constexpr int kSH = 0;
 };
-// ProjArgs with the rotation width as a compile-time constant:
-// rot_half = 32 * SH, SH = 0 .. 4.
+// The kernel argument, with the rotation width as a compile-time constant:
+// rot_half = 32 * SH, SH = 0 .. 4.  It holds the 64 SH cos / sin values in
+// use only: launch arguments are copied by the host at every call.
 template <int SH>
-struct Proj : ProjArgs {
+struct Proj : ProjInput {
   static constexpr int kSH = SH;
+  float cs[SH > 0 ? 64 * SH : 1];
 };
 template <class X>
 struct is_proj : std::false_type {};
@@ -148,7 +152,7 @@ struct is_proj<Proj<SH>> : std::true_type {};
 template <int SH>
 struct RopeTab {
   float t[SH > 0 ? SH : 1];
-  __device__ __forceinline__ void fill(const ProjArgs& x, int lane) {
+  __device__ __forceinline__ void fill(const Proj<SH>& x, int lane) {
 #pragma unroll
     for (int s = 0; s < SH; s++) {
       float v = 0.f;
@@ -194,7 +198,7 @@ struct HeadPart {
     }
   }
   template <int SH>
-  __device__ __forceinline__ void norm_rope(const ProjArgs& x, const RopeTab<SH>& tab, int lane) {
+  __device__ __forceinline__ void norm_rope(const ProjInput& x, const RopeTab<SH>& tab, int lane) {
     constexpr int TPH = D / DPT;
     const int i = lane % TPH;
     float ss = 0.f;
@@ -375,7 +379,7 @@ __device__ void merge_tail(const SplitArgs& a) {
 // sequence (with GH = 2 a workgroup reads one contiguous stretch of both
 // heads' K and V blocks).  NCB column blocks of 16 columns (column c = token
 // c / 8, query head c % 8 of the group).
-// With X = ProjArgs (decode step from projections, one token, NCB = 1) the
+// With X = Proj (decode step from projections, one token, NCB = 1) the
 // kernel also norms and rotates Q per wave, and the workgroup holding row
 // app0 norms, rotates and appends K and appends V.
 template <int NWH, int NCB, int GH, typename X, bool FLAT>
@@ -1062,7 +1066,8 @@ template <int SH>
 mi_status launch_proj(const SplitArgs& a, const SplitPlan& plan, hipStream_t stream,
                       const ProjArgs& p) {
   Proj<SH> x;
-  static_cast<ProjArgs&>(x) = p;
+  static_cast<ProjInput&>(x) = p;
+  std::copy(p.cs, p.cs + 64 * SH, x.cs);
   if (plan.gh == 2) return launch_split<4, 1, 2>(a, 1, stream, x);
   return launch_split<8, 1, 1>(a, 1, stream, x);
 }
@@ -1535,7 +1540,7 @@ extern "C" mi_status mi_attn_step_proj(mi_kv* kv, int32_t layer, const float* q_
                     "mi_qk_norm_rope_append + mi_attn_decode",
                     rotary_dim);
   MI_TRY(mi::kv_grow(kv, pos + 1, (hipStream_t)stream));
-  ProjArgs x{};
+  ProjArgs x;
   x.q_proj = q_proj;
   x.k = k;
   x.v = v;
@@ -1548,8 +1553,7 @@ extern "C" mi_status mi_attn_step_proj(mi_kv* kv, int32_t layer, const float* q_
   const float fpos = (float)pos;
   for (int i = 0; i < x.rot_half; i++) {
     const float theta = fpos * inv_freq[i];
-    x.cs[i] = cosf(theta);
-    x.cs[x.rot_half + i] = sinf(theta);
+    sincosf(theta, &x.cs[x.rot_half + i], &x.cs[i]);
   }
   const int64_t rows = pos + 1;
   const SplitPlan plan = plan_split(rows, 1, kv->G, 1);

@@ -12,6 +12,7 @@
 // (src/math_util.rs:501-593; Metal kernels src/engine/shaders.metal:2244-2363)
 // followed by kv_cache_append (math_util.rs:387-392).  K is rotated from its
 // un-rotated normed values (the CPU form's `orig` copy, math_util.rs:566).
+#include <algorithm>
 #include <cmath>
 
 #include "common.h"
@@ -121,9 +122,19 @@ mi_status check_rope(const mi_kv* kv, int32_t rotary_dim, float rope_theta, floa
   return MI_OK;
 }
 
+// A model has one (rope_theta, rotary_dim): the table of the last pair is kept
+// per thread, so a decode step does not pay 32 powf calls again (1.3 us).
 void rope_inv_freq(float rope_theta, int32_t rotary_dim, float* inv_freq) {
-  for (int i = 0; i < rotary_dim / 2; i++)
-    inv_freq[i] = powf(rope_theta, -2.0f * (float)i / (float)rotary_dim);
+  thread_local float theta = 0.f, table[kMaxRotHalf];
+  thread_local int32_t dim = -1;
+  const int half = rotary_dim / 2;
+  if (theta != rope_theta || dim != rotary_dim) {
+    for (int i = 0; i < half; i++)
+      table[i] = powf(rope_theta, -2.0f * (float)i / (float)rotary_dim);
+    theta = rope_theta;
+    dim = rotary_dim;
+  }
+  std::copy(table, table + half, inv_freq);
 }
 
 }  // namespace mi
