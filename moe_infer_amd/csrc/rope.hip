@@ -1,12 +1,18 @@
 // Per-head RMS norm + NeoX partial rotary embedding of Q and K, fused with the
 // KV-cache append of the rotated K and the raw V rows.
 //
-// One wavefront per head; lane l holds columns 4l..4l+3 of head_dim = 256.
-// Waves 0..H-1 of a token take the query heads (q_proj block [Q | gate]),
-// waves H..H+G-1 the KV heads (K norm + rope into the cache, V converted and
-// stored beside it).  The RoPE partner of column d < rotary_dim/2 is
-// d + rotary_dim/2, i.e. lane l + rotary_dim/8, fetched with a cross-lane
-// shuffle of the normed values.
+// Bound: memory (36 KiB read and 18 KiB written per token) for many tokens, the
+// chain of one wave for few.  A wave64 VALU instruction takes four clocks, so
+// four sincosf per lane and head cost more than the bytes did: a wave takes
+// one head and computes each angle once, in one lane.  K goes by 16 rows of a
+// cache block (one row half of the layout), through LDS, and leaves as whole
+// 1 KiB wave stores; V is gathered by column so that a store holds the eight
+// rows of a V block.  Row by row, K left in 8-byte and V in 2-byte pieces of
+// lines that other CUs also wrote.  Measured per call against four sincosf and
+// row-wise stores: 4096 tokens 62.6 -> 36.4 us (6.2 TB/s), 1900 tokens 27.1 ->
+// 18.5, 333 tokens 7.4 -> 5.4, 12 tokens 3.6 -> 2.7.  Two, four or eight heads
+// to a wave (more loads in flight, fewer sincosf): 1900 tokens 18.4, 19.1 and
+// 21.1 us, 12 tokens 2.9, 3.3 and 4.4.
 //
 // Reference semantics: q_head_norm_rope / k_head_norm_rope
 // (src/math_util.rs:501-593; Metal kernels src/engine/shaders.metal:2244-2363)
@@ -16,6 +22,8 @@
 #include <cmath>
 
 #include "common.h"
+
+extern "C" __device__ float __ockl_wfred_add_f32(float);
 
 namespace {
 
@@ -32,81 +40,211 @@ struct RopeArgs {
   _Float16* kc;           // cache K blocks of the layer
   _Float16* vc;           // cache V blocks of the layer
   int64_t pos;            // row of token 0
-  int H, G, rot_half;
+  int n, H, G, rot_half;
+  int nk, nkv;            // workgroups of K, of K and V
   float eps;
   // rope_theta^(-2i/rotary_dim), computed on the host in f32 with the
   // reference's expression so that theta = pos * inv_freq rounds identically.
   float inv_freq[kMaxRotHalf];
 };
 
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, 64);
-  return x;
+// K staging: the block layout of one (block, head, row half), each column
+// chunk's 16 row slots padded by 16 bytes so that a wave's 8-byte writes
+// (lanes two to a chunk) spread over the banks.
+constexpr int kChunkPitch = 16 * 8 + 8;  // halves
+constexpr int kStageHalves = 32 * kChunkPitch;
+
+// Tokens from which K goes through LDS by block; fewer go row by row, a wave
+// each, which has the shorter chain: the call takes 2.7 / 2.8 / 3.4 us for 12
+// / 64 / 128 tokens, by block 3.9 / 4.1 / 4.5.
+constexpr int kKRowTokens = 192;
+
+// RMS norm of one head, lane l holding columns 4l .. 4l+3.
+__device__ __forceinline__ void head_norm(const float4& x, const ushort4& wb, float eps,
+                                          float (&y)[4]) {
+  const float ss = __ockl_wfred_add_f32(x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w);
+  const float inv_rms = 1.0f / sqrtf(ss / (float)mi::kHeadDim + eps);
+  y[0] = x.x * inv_rms * mi::bf16_to_f32(wb.x);
+  y[1] = x.y * inv_rms * mi::bf16_to_f32(wb.y);
+  y[2] = x.z * inv_rms * mi::bf16_to_f32(wb.z);
+  y[3] = x.w * inv_rms * mi::bf16_to_f32(wb.w);
 }
 
-__global__ void __launch_bounds__(256) qk_norm_rope_kernel(const RopeArgs a) {
-  constexpr int D = mi::kHeadDim;
-  const int lane = threadIdx.x & 63;
-  const int head = blockIdx.y * 4 + (threadIdx.x >> 6);
-  const int t = blockIdx.x;
-  if (head >= a.H + a.G) return;  // whole waves
-  const bool is_q = head < a.H;
-  const int kh = head - a.H;
-  const int c0 = 4 * lane;
-
-  const float* src = is_q ? a.q_proj + ((int64_t)t * a.H + head) * (2 * D)
-                          : a.k + ((int64_t)t * a.G + kh) * D;
-  const float4 x = *(const float4*)(src + c0);
-  const uint16_t* w = is_q ? a.q_w : a.k_w;
-  const ushort4 wb = *(const ushort4*)(w + c0);
-
-  float ss = x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
-  ss = wave_sum(ss);
-  const float inv_rms = 1.0f / sqrtf(ss / (float)D + a.eps);
-
-  float y[4] = {x.x * inv_rms * mi::bf16_to_f32(wb.x), x.y * inv_rms * mi::bf16_to_f32(wb.y),
-                x.z * inv_rms * mi::bf16_to_f32(wb.z), x.w * inv_rms * mi::bf16_to_f32(wb.w)};
-
-  const int rh = a.rot_half;
-  const bool lower = c0 < rh;
+// NeoX rotation of a normed head; c, s: the lane's four angles (pairs
+// 4l mod rot_half ..), read only where 4l < 2 rot_half.
+__device__ __forceinline__ f16x4 head_rotate(float (&y)[4], const float (&c)[4],
+                                             const float (&s)[4], int lane, int rh) {
+  const bool lower = 4 * lane < rh;
   const int partner = lower ? lane + (rh >> 2) : lane - (rh >> 2);
   float pr[4];
 #pragma unroll
   for (int e = 0; e < 4; e++) pr[e] = __shfl(y[e], partner & 63, 64);
-  if (c0 < 2 * rh) {
-    const float fpos = (float)(a.pos + t);
-    const int p0 = lower ? c0 : c0 - rh;
+  if (4 * lane < 2 * rh) {
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-      const float theta = fpos * a.inv_freq[p0 + e];
-      float s, c;
-      sincosf(theta, &s, &c);
-      y[e] = lower ? y[e] * c - pr[e] * s : pr[e] * s + y[e] * c;
-    }
+    for (int e = 0; e < 4; e++)
+      y[e] = lower ? y[e] * c[e] - pr[e] * s[e] : pr[e] * s[e] + y[e] * c[e];
   }
   f16x4 h;
 #pragma unroll
   for (int e = 0; e < 4; e++) h[e] = (_Float16)y[e];
+  return h;
+}
 
-  if (is_q) {
-    const int64_t o = ((int64_t)t * a.H + head) * D + c0;
-    *(f16x4*)(a.q_out + o) = h;
-    const float4 g = *(const float4*)(src + D + c0);
-    f16x4 gh;
-    gh[0] = (_Float16)g.x;
-    gh[1] = (_Float16)g.y;
-    gh[2] = (_Float16)g.z;
-    gh[3] = (_Float16)g.w;
-    *(f16x4*)(a.gate_out + o) = gh;
-  } else {
-    const int64_t r = a.pos + t;
-    *(f16x4*)(a.kc + mi::k_offset(r, kh, c0, a.G, D)) = h;
-    const float4 vv = *(const float4*)(a.v + ((int64_t)t * a.G + kh) * D + c0);
-    const float vs[4] = {vv.x, vv.y, vv.z, vv.w};
+// The lane's four angles of token tok's rotation, computed one (BIG: two) per
+// lane and fetched from the lanes that hold them.
+template <bool BIG>
+__device__ __forceinline__ void lane_angles(const RopeArgs& a, int tok, int lane, float (&c)[4],
+                                            float (&s)[4]) {
+  const int rh = a.rot_half;
+  const float fpos = (float)(a.pos + tok);
+  float ct[BIG ? 2 : 1] = {}, st[BIG ? 2 : 1] = {};
 #pragma unroll
-    for (int e = 0; e < 4; e++) a.vc[mi::v_offset(r, kh, c0 + e, a.G, D)] = (_Float16)vs[e];
+  for (int k = 0; k < (BIG ? 2 : 1); k++)
+    if (lane + 64 * k < rh) sincosf(fpos * a.inv_freq[lane + 64 * k], &st[k], &ct[k]);
+  const int p0 = 4 * lane < rh ? 4 * lane : 4 * lane - rh;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    c[e] = __shfl(ct[0], (p0 + e) & 63, 64);
+    s[e] = __shfl(st[0], (p0 + e) & 63, 64);
+    if constexpr (BIG) {
+      const float c1 = __shfl(ct[1], (p0 + e) & 63, 64), s1 = __shfl(st[1], (p0 + e) & 63, 64);
+      if (p0 + e >= 64) {
+        c[e] = c1;
+        s[e] = s1;
+      }
+    }
   }
+}
+
+// One K row by one wave, stored in place (a few rows: kKRowTokens).
+template <bool BIG>
+__device__ __forceinline__ void k_row(const RopeArgs& a, int item) {
+  constexpr int D = mi::kHeadDim;
+  const int lane = threadIdx.x & 63;
+  const int tok = item / a.G, h = item - tok * a.G;
+  if (tok >= a.n) return;
+  const float4 x = *(const float4*)(a.k + (int64_t)item * D + 4 * lane);
+  const ushort4 wb = *(const ushort4*)(a.k_w + 4 * lane);
+  float y[4], c[4], s[4];
+  lane_angles<BIG>(a, tok, lane, c, s);
+  head_norm(x, wb, a.eps, y);
+  *(f16x4*)(a.kc + mi::k_offset(a.pos + tok, h, 4 * lane, a.G, D)) =
+      head_rotate(y, c, s, lane, a.rot_half);
+}
+
+// K rows of one (32-row block, KV head, row half u): 16 rows, four per wave,
+// whose slots are 8 KiB of contiguous block layout.  `lds`: the stage, then
+// the angles [16][rot_half] (cos, sin).  Loads are unconditional (rows outside
+// [pos, pos + n) read a row inside it and are not stored), so that all are in
+// flight before the first is waited for.
+__device__ __forceinline__ void k_rows(const RopeArgs& a, int item, float* lds) {
+  constexpr int D = mi::kHeadDim;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int u = item & 1, bh = item >> 1;
+  const int bb = bh / a.G, h = bh - bb * a.G;
+  const int64_t b = a.pos / MI_KV_KBLOCK + bb;
+  const int64_t row0 = b * MI_KV_KBLOCK - a.pos + 8 * w + 4 * u;  // token of the wave's first row
+  const int rh = a.rot_half;
+  _Float16* const stage = (_Float16*)lds;
+  float2* const tab = (float2*)(lds + kStageHalves / 2) + 4 * w * rh;
+
+  float4 x[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int64_t tok = min(max(row0 + i, (int64_t)0), (int64_t)a.n - 1);
+    x[i] = *(const float4*)(a.k + (tok * a.G + h) * D + 4 * lane);
+  }
+  const ushort4 wb = *(const ushort4*)(a.k_w + 4 * lane);
+  // the angles of the wave's new rows [i0, i1), spread over its lanes
+  const int i0 = (int)min(max(-row0, (int64_t)0), (int64_t)4);
+  const int i1 = (int)min(max((int64_t)a.n - row0, (int64_t)0), (int64_t)4);
+  for (int idx = i0 * rh + lane; idx < i1 * rh; idx += 64) {
+    const int i = (idx >= rh) + (idx >= 2 * rh) + (idx >= 3 * rh), p = idx - i * rh;
+    float sn, cs;
+    sincosf((float)(a.pos + row0 + i) * a.inv_freq[p], &sn, &cs);
+    tab[idx] = float2{cs, sn};
+  }
+  const bool rot = 4 * lane < 2 * rh;
+  const int p0 = 4 * lane < rh ? 4 * lane : 4 * lane - rh;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    float y[4], c[4], s[4];
+    head_norm(x[i], wb, a.eps, y);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {  // this wave's own table rows
+      const float2 cs = rot ? tab[i * rh + p0 + e] : float2{};
+      c[e] = cs.x;
+      s[e] = cs.y;
+    }
+    *(f16x4*)(stage + (lane >> 1) * kChunkPitch + (4 * w + i) * 8 + 4 * (lane & 1)) =
+        head_rotate(y, c, s, lane, rh);
+  }
+  __syncthreads();
+  _Float16* kd = a.kc + ((b * a.G + h) * 2 + u) * (int64_t)(16 * D);
+#pragma unroll
+  for (int i = 0; i < 2; i++) {  // slot (chunk, j), j fastest
+    const int sl = 256 * i + t, j = sl & 15;
+    const int64_t tk = b * MI_KV_KBLOCK - a.pos + (((j >> 2) << 3) | (u << 2) | (j & 3));
+    if (tk >= 0 && tk < a.n)
+      *(f16x8*)(kd + sl * 8) = *(const f16x8*)(stage + (sl >> 4) * kChunkPitch + j * 8);
+  }
+}
+
+// V rows of one (8-row block, KV head): thread t gathers column t.
+__device__ __forceinline__ void v_rows(const RopeArgs& a, int item) {
+  constexpr int D = mi::kHeadDim;
+  const int t = threadIdx.x;
+  const int bb = item / a.G, h = item - bb * a.G;
+  const int64_t b = a.pos / MI_KV_VBLOCK + bb;
+  const int64_t row0 = b * MI_KV_VBLOCK - a.pos;  // token of the block's first row
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const int64_t tok = min(max(row0 + e, (int64_t)0), (int64_t)a.n - 1);
+    x[e] = a.v[(tok * a.G + h) * D + t];
+  }
+  _Float16* vd = a.vc + (b * a.G + h) * (int64_t)(D * MI_KV_VBLOCK) + t * 8;
+  f16x8 col;
+#pragma unroll
+  for (int e = 0; e < 8; e++) col[e] = (_Float16)x[e];
+  if (row0 >= 0 && row0 + 8 <= a.n) {
+    *(f16x8*)vd = col;
+  } else {  // rows outside the range keep their contents
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      if (row0 + e >= 0 && row0 + e < a.n) vd[e] = col[e];
+  }
+}
+
+// Workgroups [0, nk): K, [nk, nkv): V blocks; then one query head of one token
+// per wave.  BIG: rot_half above 64, two angles a lane.
+template <bool BIG>
+__global__ void __launch_bounds__(256) qk_norm_rope_kernel(const RopeArgs a) {
+  constexpr int D = mi::kHeadDim;
+  extern __shared__ float lds[];
+  const int wave = threadIdx.x >> 6;
+  const int wg = blockIdx.y * gridDim.x + blockIdx.x;
+  if (wg < a.nkv) {
+    if (wg >= a.nk) v_rows(a, wg - a.nk);
+    else if (a.n < kKRowTokens) k_row<BIG>(a, wg * 4 + wave);
+    else k_rows(a, wg, lds);
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  const int64_t head = (int64_t)(wg - a.nkv) * 4 + wave;  // tok * H + head
+  const int tok = (int)(head / a.H);
+  if (tok >= a.n) return;  // whole waves
+  const float* src = a.q_proj + head * (2 * D) + 4 * lane;
+  const float4 x = *(const float4*)src;
+  const float4 g = *(const float4*)(src + D);
+  const ushort4 wb = *(const ushort4*)(a.q_w + 4 * lane);
+  float y[4], c[4], s[4];
+  lane_angles<BIG>(a, tok, lane, c, s);
+  head_norm(x, wb, a.eps, y);
+  const int64_t o = head * D + 4 * lane;
+  *(f16x4*)(a.q_out + o) = head_rotate(y, c, s, lane, a.rot_half);
+  *(f16x4*)(a.gate_out + o) =
+      f16x4{(_Float16)g.x, (_Float16)g.y, (_Float16)g.z, (_Float16)g.w};
 }
 
 }  // namespace
@@ -165,14 +303,24 @@ extern "C" mi_status mi_qk_norm_rope_append(mi_kv* kv, int32_t layer, const floa
   a.kc = kv->k[layer];
   a.vc = kv->v[layer];
   a.pos = pos;
+  a.n = n;
   a.H = kv->H;
   a.G = kv->G;
   a.rot_half = rotary_dim / 2;
   a.eps = eps;
   mi::rope_inv_freq(rope_theta, rotary_dim, a.inv_freq);
 
-  const int waves = kv->H + kv->G;
-  MI_HIP(mi::launch("qk_norm_rope", qk_norm_rope_kernel, dim3(n, (waves + 3) / 4), dim3(256), 0,
+  const int64_t last = pos + n - 1;
+  const bool by_row = n < kKRowTokens;
+  a.nk = by_row ? (n * kv->G + 3) / 4
+                : (int)(2 * (last / MI_KV_KBLOCK - pos / MI_KV_KBLOCK + 1) * kv->G);
+  a.nkv = a.nk + (int)((last / MI_KV_VBLOCK - pos / MI_KV_VBLOCK + 1) * kv->G);
+  const int64_t wgs = a.nkv + ((int64_t)n * kv->H + 3) / 4;
+  const int64_t gx = std::min<int64_t>(wgs, 1 << 22);  // a grid row is below 2^32 threads
+  const size_t lds = by_row ? 0 : kStageHalves * sizeof(_Float16) + 16 * a.rot_half * sizeof(float2);
+  MI_HIP(mi::launch("qk_norm_rope",
+                    a.rot_half > 64 ? qk_norm_rope_kernel<true> : qk_norm_rope_kernel<false>,
+                    dim3((unsigned)gx, (unsigned)((wgs + gx - 1) / gx)), dim3(256), lds,
                     (hipStream_t)stream, a));
   kv->len[layer] = pos + n;
   return MI_OK;
