@@ -205,6 +205,10 @@ mi_status verify_wide_split(const mi_kv* kv, int32_t layer, const _Float16* q, i
 // the merge (decode.hip).  out [n][H][D], optional gate [n][H][D].
 mi_status attend_wide(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
                       _Float16* out, int64_t past, int32_t n, hipStream_t stream);
+// The same in one launch (decode.hip), where n and past are in its range;
+// false (and nothing done) where they are not.
+bool attend_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
+                   _Float16* out, int64_t past, int32_t n, hipStream_t stream, mi_status* st);
 // Workspace bytes attend_wide needs for these sizes.
 size_t wide_workspace_bytes(int G, int64_t past, int32_t n);
 // Enqueues the row copy of kv_cache_append_n on `stream` (no len update).

@@ -808,6 +808,247 @@ attn_split_kernel(SplitArgs a, X x) {
   }
 }
 
+// ---- one launch for few keys per query: no chunks, no partials, no merge
+// launch.  A workgroup holds the 8 query heads of two tokens (16 columns) and
+// NDB * 16 of the 256 value columns of one KV head, and walks every key they
+// see: its four waves take 32-key tiles in turn, straight from the cache into
+// registers as in attn_split_kernel, merge through LDS, and the workgroup
+// normalises, gates and writes the output.  K(next) is requested when QK has
+// read K, V(next) when PV has read V.
+//
+// Bound: the chain launch - Q - K - QK - V - PV - merge of one workgroup, then
+// what one CU can load (~50 bytes a clock: 32 keys of K and V took 2.5 us for
+// eight waves at once).  Hence the slices of V: with NDB = 4 a decode step
+// loads K four times but on four CUs.  Four waves measured
+// best (us, 2 / 4 / 8 / 16 waves at 517 rows: 10.0 with NDB = 16 / 6.0 / 6.7 /
+// 11.8).  A step at 517 rows from HBM 10.9 -> 7.1 us, from projections 13.5 ->
+// 9.2, four draft tokens after 300 rows 14.4 -> 5.9, 64 prompt tokens 14.9 ->
+// 6.7 with their append.
+struct DirectArgs {
+  const _Float16* k;
+  const _Float16* v;
+  const _Float16* q;       // [n][H][D]
+  const _Float16* gate;    // [n][H][D] or null
+  const float* gate32;     // or the gate halves of q_proj [H][2*D], n = 1 (else null)
+  _Float16* out;           // [n][H][D]
+  const _Float16* app_k;   // rows [past, past + n) to append first ([n][G*D]), or null
+  const _Float16* app_v;
+  _Float16* kw;
+  _Float16* vw;
+  int past, n, G, H;       // token i sees keys [0, past + i]
+  float scale_log2e;
+};
+
+constexpr int kDirectWaves = 4;
+template <int NDB, typename X>
+__global__ void __launch_bounds__(kDirectWaves * 64, 2)
+attn_direct_kernel(DirectArgs a, X x) {
+  constexpr bool kProj = is_proj<X>::value;
+  constexpr int NWH = kDirectWaves, TOK = 2, NCOL = 16, SL = 16 / NDB, DS = NDB * 16;
+  extern __shared__ float smem[];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, j = lane & 15;
+  const int G = a.G;
+  const int t0 = (gridDim.x - 1 - blockIdx.x) * TOK;  // heaviest first
+  const int kvh = blockIdx.y / SL, d0 = (blockIdx.y % SL) * DS;
+  const int ntok = min(TOK, a.n - t0);
+  const int rows = a.past + t0 + ntok;  // keys the last token sees
+
+  // Appended rows: every workgroup writes the K rows of its head that its
+  // tokens see and its own value columns of V, and reads its own writes.
+  // Workgroups of one head write the same bytes to the same K rows.
+  RopeTab<X::kSH> tab;
+  constexpr int kTPH = NWH * 8;  // lanes per query head of the projection prologue
+  HeadPart<kProj ? D / kTPH : 4> qpart;
+  if constexpr (kProj) {
+    qpart.load(x.q_proj + (kvh * 8 + threadIdx.x / kTPH) * (2 * D), x.q_w, lane);
+    tab.fill(x, lane);
+    if (w == 0) {  // the whole wave (the angles are spread over it), head by its first kTPH lanes
+      constexpr int DPT = D / kTPH;
+      static_assert(kTPH <= 64, "one wave holds the K head");
+      HeadPart<DPT> kp;
+      kp.load(x.k + kvh * D, x.k_w, lane);
+      kp.template norm_rope<X::kSH>(x, tab, lane);
+      typedef _Float16 fv __attribute__((ext_vector_type(DPT)));
+      fv h;
+#pragma unroll
+      for (int e = 0; e < DPT; e++) h[e] = (_Float16)kp.y[e];
+      if (lane < kTPH) *(fv*)(a.kw + mi::k_offset(a.past, kvh, DPT * lane, G, D)) = h;
+    }
+    for (int i = threadIdx.x; i < DS; i += NWH * 64)
+      a.vw[mi::v_offset(a.past, kvh, d0 + i, G, D)] = (_Float16)x.v[kvh * D + d0 + i];
+    __syncthreads();
+  } else if (a.app_k) {
+    const int nrow = rows - a.past;
+    for (int it = threadIdx.x; it < nrow * (D / 8); it += NWH * 64) {
+      const int r = it / (D / 8), c = it % (D / 8);
+      *(f16x8*)(a.kw + mi::k_offset(a.past + r, kvh, 8 * c, G, D)) =
+          *(const f16x8*)(a.app_k + (r * G + kvh) * D + 8 * c);
+    }
+    for (int it = threadIdx.x; it < nrow * DS; it += NWH * 64) {
+      const int r = it / DS, i = d0 + it % DS;
+      a.vw[mi::v_offset(a.past + r, kvh, i, G, D)] = a.app_v[(r * G + kvh) * D + i];
+    }
+    __syncthreads();
+  }
+
+  constexpr int kRow = DS + 4;  // merge rows, padded by one 16-byte slot
+  _Float16* const qs = (_Float16*)(smem + NWH * NCOL * (kRow + 2));  // kProj: [8][kQRow]
+  constexpr int kQRow = D + 8;
+  f16x8 qf[8];
+  int lim;  // keys this lane's column sees
+  if constexpr (kProj) {
+    constexpr int DPT = D / kTPH;
+    typedef _Float16 fv __attribute__((ext_vector_type(DPT)));
+    qpart.template norm_rope<X::kSH>(x, tab, lane);
+    fv h;
+#pragma unroll
+    for (int e = 0; e < DPT; e++) h[e] = (_Float16)qpart.y[e];
+    *(fv*)(qs + (threadIdx.x / kTPH) * kQRow + DPT * (lane % kTPH)) = h;
+    mi::sync_lds();
+#pragma unroll
+    for (int kk = 0; kk < 8; kk++)
+      qf[kk] = j < 8 ? *(const f16x8*)(qs + (j & 7) * kQRow + 8 * g + 32 * kk) : f16x8{};
+    lim = j < 8 ? rows : 0;
+  } else {
+    const int tok = j >> 3;
+    const bool on = tok < ntok;
+    const _Float16* qp =
+        a.q + ((int64_t)(t0 + (on ? tok : 0)) * a.H + kvh * 8 + (j & 7)) * D + 8 * g;
+#pragma unroll
+    for (int kk = 0; kk < 8; kk++) qf[kk] = *(const f16x8*)(qp + 32 * kk);
+    lim = on ? a.past + t0 + tok + 1 : 0;  // a padding column sees no key
+  }
+
+  float m = kNegBig, l = 0.f;
+  f32x4 acc[NDB];
+#pragma unroll
+  for (int d = 0; d < NDB; d++) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f16x8 kf[2][8], vf[NDB];
+  const _Float16* const kb = a.k + (int64_t)kvh * (32 * D) + g * 128 + j * 8;
+  const _Float16* const vb = a.v + ((int64_t)g * G + kvh) * (D * 8) + (d0 + j) * 8;
+  auto load_k = [&](int t) {
+    const _Float16* kp = kb + (int64_t)t * G * (32 * D);
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int kk = 0; kk < 8; kk++) kf[u][kk] = *(const f16x8*)(kp + u * (16 * D) + kk * 512);
+  };
+  auto load_v = [&](int t) {
+    const _Float16* vp = vb + (int64_t)t * G * (32 * D);
+#pragma unroll
+    for (int d = 0; d < NDB; d++) vf[d] = *(const f16x8*)(vp + d * 128);
+  };
+  const int ntiles = (rows + 31) / 32;
+  const float c2 = a.scale_log2e;
+  if (w < ntiles) {
+    load_k(w);
+    load_v(w);
+  }
+  for (int t = w; t < ntiles; t += NWH) {
+    f32x4 st[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      f32x4 c4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < 8; kk++)
+        c4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[u][kk], qf[kk], c4, 0, 0, 0);
+      st[u] = c4;
+    }
+    if (t + NWH < ntiles) load_k(t + NWH);
+    if (32 * t + 32 > a.past + t0 + 1) {  // some column does not see the whole tile
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (32 * t + 8 * g + 4 * u + e >= lim) st[u][e] = -INFINITY;
+    }
+    float mt = fmaxf(st[0][0], st[1][0]);
+#pragma unroll
+    for (int e = 1; e < 4; e++) mt = fmaxf(mt, fmaxf(st[0][e], st[1][e]));
+    mt = mi::max_rows(mt) * c2;
+    const float mnew = fmaxf(m, mt);
+    if (__ballot(mnew != m)) {
+      const float alpha = __builtin_amdgcn_exp2f(m - mnew);
+      l *= alpha;
+#pragma unroll
+      for (int d = 0; d < NDB; d++) acc[d] *= alpha;
+      m = mnew;
+    }
+    // The row sum adds the f16 weights the PV MFMA uses.
+    float rs = 0.f;
+    f16x8 pf;
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        const f16x2 ph = {(_Float16)__builtin_amdgcn_exp2f(fmaf(st[u][e], c2, -m)),
+                          (_Float16)__builtin_amdgcn_exp2f(fmaf(st[u][e + 1], c2, -m))};
+        rs = __builtin_amdgcn_fdot2(ph, f16x2{1.f16, 1.f16}, rs, false);
+        pf[4 * u + e] = ph[0];
+        pf[4 * u + e + 1] = ph[1];
+      }
+    l += mi::sum_rows(rs);
+    if (32 * t + 32 > rows) {  // stale rows may hold anything, 0 * NaN is NaN
+      const int valid = rows - (32 * t + 8 * g);
+#pragma unroll
+      for (int d = 0; d < NDB; d++)
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          if (e >= valid) vf[d][e] = (_Float16)0.f;
+    }
+#pragma unroll
+    for (int d = 0; d < NDB; d++)
+      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[d], pf, acc[d], 0, 0, 0);
+    if (t + NWH < ntiles) load_v(t + NWH);
+  }
+
+  // merge of the waves through LDS: O [NWH][NCOL][kRow], then (m, l)
+  float* const so = smem;
+  float2* const sml = (float2*)(smem + NWH * NCOL * kRow);
+  float* dst = so + (w * NCOL + j) * kRow + 4 * g;
+#pragma unroll
+  for (int d = 0; d < NDB; d++) *(f32x4*)(dst + d * 16) = acc[d];
+  if (g == 0) sml[w * NCOL + j] = float2{m, l};
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < ntok * 8 * (DS / 4); idx += NWH * 64) {
+    const int c = idx / (DS / 4), d4 = (idx % (DS / 4)) * 4;
+    const int hq = kvh * 8 + (c & 7), tok = t0 + (c >> 3);
+    const int64_t o0 = ((int64_t)tok * a.H + hq) * D + d0 + d4;
+    f32x4 gv;
+    if (a.gate) {
+      const f16x4 gh = *(const f16x4*)(a.gate + o0);
+#pragma unroll
+      for (int e = 0; e < 4; e++) gv[e] = (float)gh[e];
+    } else if (a.gate32) {
+      gv = *(const f32x4*)(a.gate32 + hq * (2 * D) + D + d0 + d4);
+    }
+    float M = kNegBig;
+#pragma unroll
+    for (int ww = 0; ww < NWH; ww++) M = fmaxf(M, sml[ww * NCOL + c].x);
+    float L = 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ww = 0; ww < NWH; ww++) {
+      const float2 ml = sml[ww * NCOL + c];
+      const float sc = __builtin_amdgcn_exp2f(ml.x - M);
+      L += ml.y * sc;
+      o += *(const f32x4*)(so + (ww * NCOL + c) * kRow + d4) * sc;
+    }
+    // out = O / L (zero when L = 0, math_util.rs:357, 372), then the gate
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    f16x4 h;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      float r = o[e] * inv;
+      if (a.gate || a.gate32) r = mi::gate_mul(r, gv[e]);
+      h[e] = (_Float16)r;
+    }
+    *(f16x4*)(a.out + o0) = h;
+  }
+}
+
 struct CombineArgs {
   const int32_t* offsets;  // ragged (else null)
   const int32_t* lengths;  // ragged (else null)
@@ -1063,13 +1304,35 @@ mi_status launch_split(const SplitArgs& a, int64_t batch, hipStream_t stream, co
 }
 
 template <int SH>
-mi_status launch_proj(const SplitArgs& a, const SplitPlan& plan, hipStream_t stream,
-                      const ProjArgs& p) {
+Proj<SH> make_proj(const ProjArgs& p) {
   Proj<SH> x;
   static_cast<ProjInput&>(x) = p;
   std::copy(p.cs, p.cs + 64 * SH, x.cs);
+  return x;
+}
+
+template <int SH>
+mi_status launch_proj(const SplitArgs& a, const SplitPlan& plan, hipStream_t stream,
+                      const ProjArgs& p) {
+  const Proj<SH> x = make_proj<SH>(p);
   if (plan.gh == 2) return launch_split<4, 1, 2>(a, 1, stream, x);
   return launch_split<8, 1, 1>(a, 1, stream, x);
+}
+
+template <int NDB, typename X = NoProj>
+mi_status launch_direct(const DirectArgs& a, hipStream_t stream, const X& x = X()) {
+  size_t lds = (size_t)kDirectWaves * 16 * (NDB * 16 + 4 + 2) * sizeof(float);
+  if constexpr (is_proj<X>::value) lds += (size_t)8 * (D + 8) * sizeof(_Float16);
+  static std::atomic<uint64_t> lds_set{0};
+  MI_TRY(mi::set_lds_limit((const void*)attn_direct_kernel<NDB, X>, 80 * 1024, lds_set));
+  MI_HIP(mi::launch("attn_direct", attn_direct_kernel<NDB, X>, dim3((a.n + 1) / 2, a.G * (16 / NDB)),
+                    dim3(kDirectWaves * 64), lds, stream, a, x));
+  return MI_OK;
+}
+
+template <int SH>
+mi_status launch_direct_proj(const DirectArgs& a, hipStream_t stream, const ProjArgs& p) {
+  return launch_direct<4>(a, stream, make_proj<SH>(p));
 }
 
 size_t split_workspace_bytes(int64_t batch, int G, int max_chunks, int nq) {
@@ -1347,6 +1610,53 @@ mi_status wide_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float1
   return MI_OK;
 }
 
+// Whether n tokens after `past` rows take the one-launch form.
+// MI_ATTN_SPLIT_* and MI_ATTN_DECODE_MERGE (0 or 1) ask for forms of the split
+// launch, MI_ATTN_VERIFY_WIDE=0 for its 4-token groups.
+bool takes_direct(int64_t past, int32_t n, const _Float16* gate, const _Float16* out) {
+  if (((uintptr_t)gate | (uintptr_t)out) & 7) return false;  // 8-byte accesses here only
+  if (split_knobs().chunk > 0 || split_knobs().gh != 1 || split_knobs().wgs != 256) return false;
+  const char* merge = getenv("MI_ATTN_DECODE_MERGE");
+  if (n == 1 && merge && *merge) return false;
+  if (n > 4 && !verify_wide_enabled()) return false;
+  return mi::direct_rows(past, n);
+}
+
+mi_status run_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
+                     _Float16* out, int64_t past, int32_t n, hipStream_t stream,
+                     const _Float16* k_new, const _Float16* v_new, const ProjArgs* proj) {
+  DirectArgs a;
+  a.k = a.kw = kv->k[layer];
+  a.v = a.vw = kv->v[layer];
+  a.q = q;
+  a.gate = gate;
+  a.gate32 = proj ? proj->q_proj : nullptr;
+  a.out = out;
+  a.app_k = k_new;
+  a.app_v = v_new;
+  a.past = (int)past;
+  a.n = n;
+  a.G = kv->G;
+  a.H = kv->H;
+  a.scale_log2e = mi::kLog2e / sqrtf((float)D);
+  if (proj) {
+    switch (proj->rot_half / 32) {
+      case 0: return launch_direct_proj<0>(a, stream, *proj);
+      case 1: return launch_direct_proj<1>(a, stream, *proj);
+      case 2: return launch_direct_proj<2>(a, stream, *proj);
+      case 3: return launch_direct_proj<3>(a, stream, *proj);
+      default: return launch_direct_proj<4>(a, stream, *proj);
+    }
+  }
+  // Slices of V while the launch has fewer workgroups than CUs.  Measured
+  // (us, NDB = 4 / 8 / 16): no past, 64 tokens 3.6 / 4.3 / 5.7, 128 tokens 5.9 /
+  // 5.1 / 6.5, 333 tokens 15.6 / 12.5 / 11.3.
+  const int wgs = (n + 1) / 2 * kv->G;
+  if (wgs * 4 <= 256) return launch_direct<4>(a, stream);
+  if (wgs * 2 <= 256) return launch_direct<8>(a, stream);
+  return launch_direct<16>(a, stream);
+}
+
 // Verify / decode over the cache: n query tokens at positions past_pos ..
 // past_pos+n-1, rows [0, past_pos+n) already in the cache.
 // With k_new / v_new, the n new rows [past_pos, past_pos + n) are appended
@@ -1356,8 +1666,13 @@ mi_status wide_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float1
 mi_status cache_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
                        _Float16* out, int64_t past_pos, int32_t n, hipStream_t stream,
                        const _Float16* k_new = nullptr, const _Float16* v_new = nullptr) {
-  if (n > 4 && verify_wide_enabled())
-    return wide_attend(kv, layer, q, gate, out, past_pos, n, stream, k_new, v_new);
+  const bool direct = takes_direct(past_pos, n, gate, out);
+  if (n > 4 && verify_wide_enabled()) {
+    if (!direct) return wide_attend(kv, layer, q, gate, out, past_pos, n, stream, k_new, v_new);
+    void* ws;  // as below
+    MI_TRY(mi::kv_workspace(kv, wide_launch(kv->G, past_pos, n).ws_bytes, stream, &ws));
+    return run_direct(kv, layer, q, gate, out, past_pos, n, stream, k_new, v_new, nullptr);
+  }
   const int64_t lim0 = past_pos + 1;
   // The workspace is grown once, to the largest group's need, before any
   // launch: a growth refused under graph capture then leaves nothing of
@@ -1370,6 +1685,10 @@ mi_status cache_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float
   }
   void* ws;
   MI_TRY(mi::kv_workspace(kv, need, stream, &ws));
+  // (The one-launch form needs none, but a later captured call may count on
+  // the workspace that an eager call of this size leaves.)
+  if (direct)
+    return run_direct(kv, layer, q, gate, out, past_pos, n, stream, k_new, v_new, nullptr);
   for (int32_t t0 = 0; t0 < n; t0 += 4) {
     const int nq = (n - t0) < 4 ? (n - t0) : 4;
     const int64_t rows = past_pos + t0 + nq;  // rows the last token of this group sees
@@ -1430,6 +1749,13 @@ bool xcd_round_robin() {
 mi_status attend_cache(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
                        _Float16* out, int64_t past_pos, int32_t n, hipStream_t stream) {
   return cache_attend(kv, layer, q, gate, out, past_pos, n, stream);
+}
+
+bool attend_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
+                   _Float16* out, int64_t past, int32_t n, hipStream_t stream, mi_status* st) {
+  if (!takes_direct(past, n, gate, out)) return false;
+  *st = run_direct(kv, layer, q, gate, out, past, n, stream, nullptr, nullptr, nullptr);
+  return true;
 }
 
 mi_status attend_wide(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
@@ -1559,6 +1885,12 @@ extern "C" mi_status mi_attn_step_proj(mi_kv* kv, int32_t layer, const float* q_
   const SplitPlan plan = plan_split(rows, 1, kv->G, 1);
   void* ws;
   MI_TRY(mi::kv_workspace(kv, attend_workspace_bytes(kv->G, plan.max_chunks, 1), (hipStream_t)stream, &ws));
+  if (takes_direct(pos, 1, nullptr, (const _Float16*)out)) {
+    MI_TRY(run_direct(kv, layer, nullptr, nullptr, (_Float16*)out, pos, 1, (hipStream_t)stream,
+                      nullptr, nullptr, &x));
+    kv->len[layer] = pos + 1;
+    return MI_OK;
+  }
   AppendRows app;
   app.row0 = pos;
   app.n = 1;

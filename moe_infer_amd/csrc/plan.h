@@ -152,6 +152,19 @@ inline WidePlan wide_plan(int G, int64_t past, int n) {
   return p;
 }
 
+// Whether n query tokens after `past` rows are served by the one-launch form
+// (attn_direct_kernel).  Its time grows with the rows one workgroup walks; the
+// split launches cost about 10 us whatever the length.  Measured from HBM (us,
+// one launch against the split forms): 1 token at 517 rows 7.1 / 10.9, at 1000
+// 9.4 / 10.8, at 1100 13.2 / 10.9; 4 tokens at 1000 9.7 / 15.5, at 1500 16.1 /
+// 14.4; 8 tokens at 1500 15.5 / 19.7, at 2000 19.7 / 17.5; 16 tokens at 2000
+// 19.5 / 24.4, at 2500 23.4 / 27.0, at 3000 27.0 / 25.1.  More tokens, against
+// the prefill grid: 64 after 500 rows 11.2 / 28.0, 333 from none 15.4 / 24.8.
+inline bool direct_rows(int64_t past, int32_t n) {
+  const int64_t rows = past + n;
+  return rows <= 1024 + (n <= 16 ? 80 * (n - 1) : 0);
+}
+
 struct SplitKnobs {
   int gh;     // KV heads per workgroup (2, or 1 when set to 1)
   int wgs;    // target workgroup count

@@ -662,6 +662,11 @@ extern "C" mi_status mi_attn_prefill(mi_kv* kv, int32_t layer, const mi_f16* q,
     kv->len[layer] = past_pos + n;
   }
   hipStream_t s = (hipStream_t)stream;
+  mi_status st;
+  if (prefill_qpw() == 64 &&
+      mi::attend_direct(kv, layer, (const _Float16*)q, (const _Float16*)gate, (_Float16*)out,
+                        past_pos, n, s, &st))
+    return st;
   // A few tokens after a long past: the prefill grid (one workgroup per 128
   // queries and head) would leave most CUs idle while each of its
   // workgroups walks the whole past; the split-K form of the same tiles
