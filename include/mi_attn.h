@@ -154,7 +154,8 @@ mi_status mi_kv_copy_from(mi_kv* dst, const mi_kv* src);
 /* Decode attention of one query token over rows [0, seq_len) of `layer`:
  * out[h] = softmax(q_h . K^T / sqrt(D)) V  for every query head h, KV head
  * h / (H/G); then out *= sigmoid(gate) elementwise when gate != NULL.
- * q, gate, out: [H*D] f16.  Split-K flash-decoding plus a combine kernel.
+ * q, gate, out: [H*D] f16.  Split-K flash-decoding plus a combine kernel, or
+ * one launch up to 1024 rows.
  * Semantics: attention_scores/softmax/values_batched + sigmoid_gate_inplace
  * (src/math_util.rs:264-269, 323-383), kernels attn_sdpa_block +
  * attn_sdpa_reduce (src/engine/shaders.metal:1559-1776).  seq_len == 0 gives
@@ -176,12 +177,13 @@ mi_status mi_attn_step(mi_kv* kv, int32_t layer, const mi_f16* q,
  * batched.rs:233-260; kernels kv_cache_append_n + attn_sdpa_causal_n,
  * shaders.metal:2656-2792): append n rows k, v [n][G*D] at past_pos, then
  * query i (q [n][H][D]) attends rows [0, past_pos + i] inclusive; gate
- * [n][H][D] or NULL; out [n][H][D].  MFMA flash-attention kernel; up to
- * 1024 new tokens after a past of at least 2048 rows (and twice n) run its
- * split-K form over key chunks plus a merge, which needs the handle's
- * workspace (grown on demand; under graph capture only when it already
- * suffices, else the unsplit kernel runs).  MI_ATTN_PREFILL_SPLIT=0 turns
- * the split-K form off.
+ * [n][H][D] or NULL; out [n][H][D].  Short prompts (n (past + n/2) up to
+ * 480000, 3200 rows) run in one launch; up to 1024 new tokens after a past of
+ * at least n rows (n/2 for up to 640) the split-K form of the MFMA
+ * flash-attention kernel over key chunks plus a merge, which needs the
+ * handle's workspace (grown on demand; under graph capture only when it already
+ * suffices, else the unsplit kernel runs); anything else the unsplit kernel.
+ * MI_ATTN_PREFILL_SPLIT=0 turns the split-K form off.
  * k = v = NULL: rows [past_pos, past_pos+n) are already in the cache (written
  * by mi_qk_norm_rope_append or mi_kv_append; len(layer) >= past_pos + n), no
  * append; len(layer) becomes past_pos + n. */
@@ -195,7 +197,8 @@ mi_status mi_attn_prefill(mi_kv* kv, int32_t layer, const mi_f16* q,
  * split-K over the cache: up to 4 tokens in the decode kernel's form, more
  * in one pass of the prefill's MFMA tiles over key chunks that reads each
  * K/V tile once per 16 tokens (MI_ATTN_VERIFY_WIDE=0 runs them as 4-token
- * groups instead), then a merge.  Rollback afterwards is
+ * groups instead), then a merge; short contexts (1024 + 80 (n - 1) rows for up
+ * to 16 tokens) in one launch.  Rollback afterwards is
  * mi_kv_set_pos.  k = v = NULL as for mi_attn_prefill. */
 mi_status mi_attn_verify(mi_kv* kv, int32_t layer, const mi_f16* q,
                          const mi_f16* k, const mi_f16* v, const mi_f16* gate,

@@ -1062,6 +1062,7 @@ struct CombineArgs {
   const int32_t* tile_off;  // flat ragged split (SplitArgs::tile_off), else null
   int nwg, batch;           // flat: the split launch's gridDim.x; sequences
   int64_t nslots;           // partial slots per KV head (SplitArgs::nslots)
+  bool wide;                // partials of the wide pass: a token's are those its row block wrote
 };
 
 // Chunk merge.  One workgroup per (column, KV head x slice of S values of
@@ -1103,6 +1104,7 @@ attn_combine_kernel(CombineArgs a) {
     bad = len < 0 || len > a.kv_len || off < 0 || (off & 31);
     if (bad) len = 0;
   }
+  if (a.wide) len = mi::wide_end((int)len - a.nq, a.nq, c >> 7);
   const int nch = (int)((len + a.chunk - 1) / a.chunk);
   const int64_t base = (int64_t)s * a.max_chunks;  // first partial slot of s
   const float* ml = a.part_ml + ((kvh * a.nslots + base) * ncols + c) * 2;  // chunk ch at ml[ch * mstride]
@@ -1490,6 +1492,7 @@ mi_status run_split(const _Float16* k, const _Float16* v, const int32_t* offsets
   c.nslots = a.nslots;
   c.nwg = nwg;
   c.batch = (int)batch;
+  c.wide = false;
   if (lengths) {
     MI_HIP(mi::launch("attn_combine", attn_combine_flat_kernel, dim3(8, G, (unsigned)batch),
                       dim3(D), 0, stream, c));
@@ -1505,45 +1508,63 @@ mi_status run_split(const _Float16* k, const _Float16* v, const int32_t* offsets
   return MI_OK;
 }
 
-// Merge of a few chunks (at most kColsChunks) for many columns: one thread
-// per output value, one workgroup of D threads per (column, KV head).  The
-// wide verify's partials for many tokens come in few chunks, where
-// attn_combine_kernel's workgroup per column and 32-value slice (chunks
-// spread over its threads) would launch 16 workgroups per column.
-constexpr int kColsChunks = 16;
-__global__ void __launch_bounds__(D) attn_combine_cols_kernel(CombineArgs a) {
-  const int c = blockIdx.x, kvh = blockIdx.y, d = threadIdx.x;
+// Merge for many columns: a wave per column, four values of d per lane, so
+// that a wave reads each chunk's 1 KiB row of O in one instruction.  Columns
+// are (token, head) pairs; a token's partials are those of its row block of
+// the wide pass: chunks [0, nch), nch from the block's last key.  Used where
+// there are few chunks or many columns; attn_combine_kernel spreads the chunks
+// of a column over a workgroup instead.  Bound: the partials' bytes.  512 tokens
+// in 4 chunks (38 MB): 8.0 us = 4.7 TB/s, against 14.2 us for a thread per
+// output value with 4-byte loads.
+constexpr int kRowsBatch = 8;
+__global__ void __launch_bounds__(256) attn_combine_rows_kernel(CombineArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int c = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int kvh = blockIdx.y;
   const int ncols = a.nq * 8;
-  const int nch = (int)((a.kv_len + a.chunk - 1) / a.chunk);
-  float m[kColsChunks], l[kColsChunks], o[kColsChunks];
+  const int tok = c >> 3, hq = kvh * 8 + (c & 7);
+  const int nch = (mi::wide_end((int)a.kv_len - a.nq, a.nq, tok >> 4) + a.chunk - 1) / a.chunk;
+  const int64_t oidx = ((int64_t)tok * a.H + hq) * D + 4 * lane;
+  f16x4 gv = {};
+  if (a.gate) gv = *(const f16x4*)(a.gate + oidx);
+  const float* ml = a.part_ml + ((int64_t)kvh * a.nslots * ncols + c) * 2;
+  const float* po = a.part_o + ((int64_t)kvh * a.nslots * ncols + c) * D + 4 * lane;
+  float M = kNegBig, L = 0.f;
+  f32x4 O = {0.f, 0.f, 0.f, 0.f};
+  for (int c0 = 0; c0 < nch; c0 += kRowsBatch) {
+    float m[kRowsBatch], l[kRowsBatch];
+    f32x4 o[kRowsBatch];
 #pragma unroll
-  for (int ch = 0; ch < kColsChunks; ch++) {
-    m[ch] = kNegBig;
-    l[ch] = 0.f;
-    o[ch] = 0.f;
-    if (ch < nch) {
-      const int64_t slot = ((int64_t)kvh * a.nslots + ch) * ncols + c;
-      m[ch] = a.part_ml[slot * 2];
-      l[ch] = a.part_ml[slot * 2 + 1];
-      o[ch] = a.part_o[slot * D + d];
+    for (int k = 0; k < kRowsBatch; k++) {
+      const int64_t ch = c0 + k < nch ? c0 + k : c0;  // (a repeat is not used)
+      m[k] = ml[ch * ncols * 2];
+      l[k] = ml[ch * ncols * 2 + 1];
+      o[k] = *(const f32x4*)(po + ch * ncols * D);
+    }
+    float mx = M;
+#pragma unroll
+    for (int k = 0; k < kRowsBatch; k++) mx = fmaxf(mx, m[k]);
+    const float r = exp2f(M - mx);
+    L *= r;
+    O *= r;
+    M = mx;
+#pragma unroll
+    for (int k = 0; k < kRowsBatch; k++) {
+      const float w = c0 + k < nch ? exp2f(m[k] - M) : 0.f;
+      L += l[k] * w;
+      O += o[k] * w;
     }
   }
-  float M = kNegBig;
-#pragma unroll
-  for (int ch = 0; ch < kColsChunks; ch++) M = fmaxf(M, m[ch]);
-  float L = 0.f, O = 0.f;
-#pragma unroll
-  for (int ch = 0; ch < kColsChunks; ch++) {
-    const float w = exp2f(m[ch] - M);
-    L += l[ch] * w;
-    O += o[ch] * w;
-  }
   // out = O / L (zero when L = 0, math_util.rs:357, 372), then the gate
-  float r = (L > 0.f) ? O / L : 0.f;
-  const int tok = c >> 3, hq = kvh * 8 + (c & 7);
-  const int64_t oidx = ((int64_t)tok * a.H + hq) * D + d;
-  if (a.gate) r = mi::gate_mul(r, (float)a.gate[oidx]);
-  a.out[oidx] = (_Float16)r;
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  f16x4 h;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    float r = O[e] * inv;
+    if (a.gate) r = mi::gate_mul(r, (float)gv[e]);
+    h[e] = (_Float16)r;
+  }
+  *(f16x4*)(a.out + oidx) = h;
 }
 
 // Wide verify for more than 4 query tokens (MI_ATTN_VERIFY_WIDE=0, read at
@@ -1601,8 +1622,12 @@ mi_status wide_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float1
   c.max_chunks = nchunks;
   c.batch = 1;
   c.nslots = nchunks;
-  if (nchunks <= kColsChunks)
-    MI_HIP(mi::launch("attn_combine", attn_combine_cols_kernel, dim3(n * 8, G), dim3(D), 0,
+  c.wide = true;
+  // 16-byte lanes per column fill the CUs from 64 tokens on; for fewer with
+  // many chunks (16 tokens at 65536 rows: 114) a workgroup per column and
+  // 32-value slice does.  The rows form moves 8-byte pieces of gate and out.
+  if ((nchunks <= 16 || n >= 64) && !(((uintptr_t)gate | (uintptr_t)out) & 7))
+    MI_HIP(mi::launch("attn_combine", attn_combine_rows_kernel, dim3(n * 2, G), dim3(256), 0,
                       stream, c));
   else
     MI_HIP(mi::launch("attn_combine", attn_combine_kernel<32>, dim3(n * 8, G * (D / 32), 1),
@@ -1622,9 +1647,17 @@ bool takes_direct(int64_t past, int32_t n, const _Float16* gate, const _Float16*
   return mi::direct_rows(past, n);
 }
 
+// Most new rows the one-launch form appends itself (every workgroup of a head
+// writes them); more go in a launch before it.
+constexpr int kDirectAppend = 16;
+
 mi_status run_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
                      _Float16* out, int64_t past, int32_t n, hipStream_t stream,
                      const _Float16* k_new, const _Float16* v_new, const ProjArgs* proj) {
+  if (k_new && n > kDirectAppend) {
+    MI_TRY(mi::kv_append_rows(kv, layer, k_new, v_new, past, n, stream));
+    k_new = v_new = nullptr;
+  }
   DirectArgs a;
   a.k = a.kw = kv->k[layer];
   a.v = a.vw = kv->v[layer];

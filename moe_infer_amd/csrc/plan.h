@@ -129,23 +129,92 @@ MI_HD inline WaveTiles split_wave_tiles(int64_t begin, int64_t end, int nwh, int
 // Most chunks (partials) per sequence of one split launch.
 constexpr int kMaxSplitChunks = 1024;
 
-// Chunking of the wide verify / split-K prefill (attn_verify_wide_kernel):
-// about 256 workgroups of (row block of 16 tokens, chunk, KV head) over rows
-// [0, past + n); whole 64-key tiles; at most kMaxSplitChunks chunks (the
-// merge kernels' limit).
+// The wide verify / split-K prefill (attn_verify_wide_kernel): one workgroup
+// per KV head, row block rb of 16 tokens and chunk c that holds keys the
+// block's tokens see, rows [0, end(rb)).  Whole chunks come first, then every
+// block's last chunk, the longest first where there are several of a length: a
+// workgroup's time is its keys, and the launch ends with its last one.
+MI_HD inline int wide_end(int past, int n, int rb) {
+  return past + (n < 16 * rb + 16 ? n : 16 * rb + 16);
+}
+// Row blocks with a whole chunk c and keys after it: [wide_first(c), nrb).
+MI_HD inline int wide_first(int past, int n, int chunk, int c) {
+  const int nrb = (n + 15) / 16;
+  const int x = (int)((int64_t)(c + 1) * chunk - past);  // new tokens up to the chunk's end
+  if (x >= n) return nrb;
+  return x <= 0 ? 0 : x / 16;
+}
+MI_HD inline int wide_count(int past, int n, int chunk) {  // workgroups
+  const int nrb = (n + 15) / 16;
+  int c = past / chunk;  // chunks whole for every block
+  int items = c * nrb + nrb;
+  for (; wide_first(past, n, chunk, c) < nrb; c++) items += nrb - wide_first(past, n, chunk, c);
+  return items;
+}
+// Grid indices wide_item takes: the last chunks may leave holes among theirs.
+MI_HD inline int wide_items(int past, int n, int chunk) {
+  const int nrb = (n + 15) / 16, per = chunk / 16;
+  return wide_count(past, n, chunk) + (nrb <= per ? 0 : (nrb + per - 1) / per * per - nrb);
+}
+// Item idx of [0, wide_items): its row block and chunk; false for none.  (One
+// block, a verify of up to 16 tokens: the divisions below would cost it 0.25 of
+// 27 us.)
+MI_HD inline bool wide_item(int past, int n, int chunk, int idx, int& rb, int& c) {
+  if (n <= 16) {
+    rb = 0;
+    c = idx;
+    return true;
+  }
+  const int nrb = (n + 15) / 16, per = chunk / 16;
+  int cc = past / chunk;
+  if (idx < cc * nrb) {
+    c = idx / nrb;
+    rb = nrb - 1 - (idx - c * nrb);
+    return true;
+  }
+  idx -= cc * nrb;
+  for (;; cc++) {
+    const int first = wide_first(past, n, chunk, cc);
+    if (first >= nrb) break;
+    if (idx < nrb - first) {
+      c = cc;
+      rb = nrb - 1 - idx;
+      return true;
+    }
+    idx -= nrb - first;
+  }
+  if (nrb <= per) {
+    rb = nrb - 1 - idx;
+  } else {  // several runs of `per` blocks: the same place of each run in turn
+    const int runs = (nrb + per - 1) / per;
+    const int place = per - 1 - idx / runs;
+    rb = idx % runs * per + (place + per - past / 16 % per) % per;
+  }
+  if (rb >= nrb) return false;
+  c = (wide_end(past, n, rb) - 1) / chunk;
+  return true;
+}
+
+// Its chunking: whole 64-key tiles, at most kMaxSplitChunks chunks (the merge
+// kernels' limit), and the smallest chunk whose workgroups all run at once (256
+// CUs): one more than that waits for a whole chunk.  Measured after 1000 rows,
+// 1000 tokens: chunks of 704 keys (more than 256 workgroups) 68 us, of 1024
+// (250) 53; after 2000 rows, 500 tokens: 448 keys 60, 640 (256) 42, 832 44.
+// More than 16 (256 / G) tokens cannot fit: one chunk.
 struct WidePlan {
   int64_t chunk;
   int nchunks;
 };
 inline WidePlan wide_plan(int G, int64_t past, int n) {
-  const int64_t rows = past + n;
-  const int64_t nrb = (n + 15) / 16;
-  int64_t target = (256 + G * nrb - 1) / (G * nrb);
-  if (target < 1) target = 1;
-  int64_t chunk = (rows + target - 1) / target;
+  const int64_t rows = past + n, nrb = ((int64_t)n + 15) / 16;
+  const int64_t most = nrb * G > 256 ? nrb : 256 / G;  // workgroups per KV head
+  const int64_t keys = nrb * past + 8 * nrb * (nrb + 1);  // at least about this many to deal out
+  int64_t chunk = keys / most;
   const int64_t min_chunk = (rows + kMaxSplitChunks - 1) / kMaxSplitChunks;
   if (chunk < min_chunk) chunk = min_chunk;
   chunk = (chunk + kPrefillBK - 1) / kPrefillBK * kPrefillBK;
+  if (chunk < kPrefillBK) chunk = kPrefillBK;
+  while (chunk < rows && wide_count((int)past, n, (int)chunk) > most) chunk += kPrefillBK;
   WidePlan p;
   p.chunk = chunk;
   p.nchunks = (int)((rows + chunk - 1) / chunk);
@@ -153,16 +222,33 @@ inline WidePlan wide_plan(int G, int64_t past, int n) {
 }
 
 // Whether n query tokens after `past` rows are served by the one-launch form
-// (attn_direct_kernel).  Its time grows with the rows one workgroup walks; the
-// split launches cost about 10 us whatever the length.  Measured from HBM (us,
-// one launch against the split forms): 1 token at 517 rows 7.1 / 10.9, at 1000
-// 9.4 / 10.8, at 1100 13.2 / 10.9; 4 tokens at 1000 9.7 / 15.5, at 1500 16.1 /
-// 14.4; 8 tokens at 1500 15.5 / 19.7, at 2000 19.7 / 17.5; 16 tokens at 2000
-// 19.5 / 24.4, at 2500 23.4 / 27.0, at 3000 27.0 / 25.1.  More tokens, against
-// the prefill grid: 64 after 500 rows 11.2 / 28.0, 333 from none 15.4 / 24.8.
+// (attn_direct_kernel).  Its time grows with the rows one workgroup walks and,
+// once the CUs are taken, with the keys of all tokens; the split launches cost
+// about 10 us whatever the length.
+// Up to 16 tokens, measured from HBM (us, one launch against the split forms):
+// 1 token at 517 rows 7.1 / 10.9, at 1000 9.4 / 10.8, at 1100 13.2 / 10.9; 4
+// tokens at 1000 9.7 / 15.5, at 1500 16.1 / 14.4; 8 at 1500 15.5 / 19.7, at
+// 2000 19.7 / 17.5; 16 at 2000 19.5 / 24.4, at 3000 27.0 / 25.1.
+// More tokens, without their append (against the prefill grid / the split-K
+// pass): 64 after 1000 rows 10.4 / 35.3 / 24.2, 128 after 3000 27.8 / 82.2 /
+// 28.9, 400 after 1000 30.3 / 45.1 / 32.8, 777 from none 25.5 / 30.9 / 42.3;
+// past the line: 300 after 1500 35.3 / 53.6 / 31.5, 1024 from none 36.6 / 37.0
+// / 36.6, 17 after 5000 33.6 / 119.7 / 25.0.
 inline bool direct_rows(int64_t past, int32_t n) {
   const int64_t rows = past + n;
-  return rows <= 1024 + (n <= 16 ? 80 * (n - 1) : 0);
+  if (n <= 16) return rows <= 1024 + 80 * (n - 1);
+  return rows <= 3200 && n * (past + n / 2) <= 480000;
+}
+
+// Whether a prefill outside that takes the split-K pass and its merge rather
+// than the prefill grid (one workgroup per 128 queries and head): the grid is
+// short of workgroups and each walks the whole past.  Measured, split-K
+// against the grid (us): 512 tokens after 1000 rows 42.8 / 48.4, 640 after 600
+// 35.0 / 42.9, 1024 after 1024 53 / 62, 512 after 16384 152 / 377; it loses
+// with 1024 after 600 (57 / 53) and from none (36.6 / 37.0 at 1024 tokens, 54 /
+// 50 at 1500), and beyond 1024 tokens, which leave no CU idle.
+inline bool prefill_split_rows(int64_t past, int32_t n) {
+  return n <= 1024 && past >= (n <= 640 ? n / 2 : n);
 }
 
 struct SplitKnobs {

@@ -580,19 +580,12 @@ mi_status launch_verify_wide(const PrefillArgs& a, const VerifyArgs& v, int grid
 }
 
 // Whether mi_attn_prefill takes the split-K form (the wide verify's pass and
-// merge): up to 1024 new tokens after a past of at least 2048 rows and
-// twice the new tokens.  Timed, split-K against the prefill grid (µs):
-// past 65536: 16 / 128 / 1024 new tokens 49 / 164 / 1004 against 1434 /
-// 1446 / 1489; past 4096: 64 / 256 / 1024 tokens 36 / 47 / 115 against 105 /
-// 114 / 136; past 2048, 512 tokens 51 against 70.  It loses where the past
-// is short next to n (past 1024, 1024 tokens: 70 against 62; no past, 256
-// tokens: 32 against 20) and beyond 1024 tokens (past 32768, 1536 tokens:
-// 932 against 846).  MI_ATTN_PREFILL_SPLIT=0 (read at each call) turns it
-// off.
+// merge; mi::prefill_split_rows).  MI_ATTN_PREFILL_SPLIT=0 (read at each call)
+// turns it off.
 bool prefill_split_k(int64_t past, int32_t n) {
   const char* e = getenv("MI_ATTN_PREFILL_SPLIT");
   if (e && *e && atoi(e) == 0) return false;
-  return n <= 1024 && past >= 2048 && past >= 2 * (int64_t)n;
+  return mi::prefill_split_rows(past, n);
 }
 
 // Queries per wave of the prefill kernel: 64 (attn_prefill64_kernel, the
@@ -610,10 +603,9 @@ namespace mi {
 mi_status verify_wide_split(const mi_kv* kv, int32_t layer, const _Float16* q, int64_t past,
                             int32_t n, int64_t chunk, int32_t nchunks, float* part_o,
                             float* part_ml, hipStream_t stream) {
-  const int nrb = (n + 15) / 16;  // row blocks of 16 tokens
   if (n <= 0 || chunk <= 0 || chunk % BK != 0 || nchunks <= 0 ||
       (int64_t)nchunks * chunk < past + n || past + n + 2 * BK >= ((int64_t)1 << 31) ||
-      (int64_t)nrb * nchunks * kv->G >= ((int64_t)1 << 31))
+      ((int64_t)n + 15) / 16 * nchunks * kv->G >= ((int64_t)1 << 30))
     return fail(MI_ERR_INVALID_ARG, "verify split: n=%d chunk=%lld nchunks=%d past=%lld", n,
                 (long long)chunk, nchunks, (long long)past);
   PrefillArgs a{};
@@ -632,7 +624,7 @@ mi_status verify_wide_split(const mi_kv* kv, int32_t layer, const _Float16* q, i
   vx.nslots = nchunks;
   vx.part_o = part_o;
   vx.part_ml = part_ml;
-  return launch_verify_wide(a, vx, nrb * nchunks * kv->G, stream);
+  return launch_verify_wide(a, vx, wide_items((int)past, n, (int)chunk) * kv->G, stream);
 }
 
 }  // namespace mi

@@ -22,6 +22,7 @@
 // merges at most that many).
 #include <cstdio>
 #include <initializer_list>
+#include <vector>
 
 #include "plan.h"
 
@@ -94,7 +95,7 @@ static long long prefill64_violations(int past, int n, long long cap) {
 
 // The wide verify / split-K prefill (attn_verify_wide_kernel): plan
 // mi::wide_plan (two KV heads); workgroup (row block rb of 16 tokens, chunk
-// c): keys from kbeg = c * chunk, wave (qb, kp) walking mi::verify_wave64's
+// c), enumerated by mi::wide_item: keys from kbeg = c * chunk, wave (qb, kp) walking mi::verify_wave64's
 // tiles with the 64-query kernel's copies (K(0) first; then K(min(t + 1,
 // nt - 1)) and V(t) at tile 0 and on active tiles, else K(t + 1) when
 // t + 1 < nt and V(t); the max pass copies K only), tile T being rows
@@ -108,9 +109,17 @@ static long long wide_violations(long long past, int n, long long cap) {
   if (wp.chunk % mi::kPrefillBK || wp.nchunks > mi::kMaxSplitChunks ||
       (long long)wp.nchunks * wp.chunk < past + n)
     bad++;
+  // the items name every (row block, chunk) with visible keys exactly once
   const int nrb = (n + 15) / 16;
-  for (int rb = 0; rb < nrb; rb++)
-    for (int c = 0; c < wp.nchunks; c++) {
+  std::vector<char> named((size_t)nrb * wp.nchunks, 0);
+  const int items = mi::wide_items((int)past, n, (int)wp.chunk);
+  for (int i = 0; i < items; i++) {
+      int rb, c;
+      if (!mi::wide_item((int)past, n, (int)wp.chunk, i, rb, c)) continue;
+      if (rb < 0 || rb >= nrb || c < 0 || c >= wp.nchunks || named[(size_t)rb * wp.nchunks + c]++) {
+        bad++;
+        continue;
+      }
       const long long kbeg = (long long)c * wp.chunk;
       auto copy = [&](int T) {
         if (kbeg + (long long)T * mi::kPrefillBK + mi::kPrefillBK > cap) bad++;
@@ -138,7 +147,12 @@ static long long wide_violations(long long past, int n, long long cap) {
           if (vis_end > kbeg && vis_end > kbeg + p.kv_len) bad++;
         }
       }
-    }
+  }
+  for (int rb = 0; rb < nrb; rb++)
+    for (int c = 0; c < wp.nchunks; c++)
+      if (named[(size_t)rb * wp.nchunks + c] !=
+          ((long long)c * wp.chunk < mi::wide_end((int)past, n, rb)))
+        bad++;
   return bad;
 }
 

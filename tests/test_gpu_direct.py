@@ -52,14 +52,14 @@ def test_step(past):
 
 
 @pytest.mark.parametrize("past,n", [(0, 2), (31, 3), (500, 4), (1260, 4), (1261, 4), (97, 5),
-                                    (2208, 16), (2209, 16)])
+                                    (2208, 16), (2209, 16), (300, 40)])
 def test_verify(past, n):
     out, ref = causal_case(past, n, attn_verify)
     assert_close(out, ref, f"verify past={past} n={n}")
 
 
 @pytest.mark.parametrize("past,n", [(0, 17), (0, 64), (7, 65), (100, 128), (33, 129), (0, 333),
-                                    (700, 299)])
+                                    (700, 299), (3000, 30), (3183, 17), (500, 511)])
 def test_prefill(past, n):
     out, ref = causal_case(past, n, attn_prefill)
     assert_close(out, ref, f"prefill past={past} n={n}")
@@ -129,3 +129,24 @@ def test_same_as_the_split_forms(monkeypatch, n):
     monkeypatch.setenv("MI_ATTN_DECODE_MERGE", "0")
     monkeypatch.setenv("MI_ATTN_VERIFY_WIDE", "0")
     assert_close(one, host(call()), f"direct against split n={n}", atol=2.0 ** -10)
+
+
+@pytest.mark.parametrize("past,n", [(999, 513), (320, 640), (1030, 1024)])
+def test_split_k_with_row_blocks_of_different_length(monkeypatch, past, n):
+    """The split-K prefill where the blocks of 16 tokens see different numbers
+    of chunks: against the prefill grid (the bound of that comparison in
+    test_gpu_prefill) and, at rows on both sides of a block, the oracle."""
+    rng = np.random.default_rng(past + n)
+    rows = past + n
+    k, v = f16(rng, rows, G * D), f16(rng, rows, G * D)
+    q, g = f16(rng, n, H, D), f16(rng, n, H, D)
+    c = Cache(num_layers=1, capacity=rows)
+    c.upload(0, k[:past], v[:past])
+    announce(f"split-K rows past={past} n={n}")
+    args = (c, 0, dev(q), dev(k[past:]), dev(v[past:]), past)
+    out = host(attn_prefill(*args, gate=dev(g)))
+    monkeypatch.setenv("MI_ATTN_PREFILL_SPLIT", "0")
+    assert_close(out, host(attn_prefill(*args, gate=dev(g))), "split-K against the grid", atol=1e-3)
+    for i in (0, 15, 16, n // 2, n - 1):
+        ref = O.decode(q[i], k[:past + i + 1], v[:past + i + 1], past + i + 1, gate=g[i])
+        assert_close(out[i].reshape(-1), ref.reshape(-1), f"split-K row {i}")
