@@ -43,6 +43,16 @@ constexpr float kNegBig = -1e30f;
 // computes itself (no plan launch); larger batches run ragged_plan_kernel.
 constexpr int kFusedPlan = 256;
 
+// Ragged batches of up to kChunkTiles tiles per spare workgroup (grid minus
+// sequences) are dealt out by chunks of one sequence, ceil(tiles / spare) tiles
+// each, so that no workgroup crosses into a second sequence: a crossing runs
+// the whole chain (Q, K, V, merge, store) twice, and with a tile or two per
+// wave that chain is the launch.  Per call
+// (us, against tiles dealt evenly across sequences): 8 sequences of 100..3000
+// rows 25.7 -> 15.5, 2 of 3000 32.5 -> 15.7, 32 of 500..2000 26.4 -> 24.5, 100 of
+// 50..200 24.7 -> 18.1.
+constexpr int kChunkTiles = 16;
+
 struct SplitArgs {
   const _Float16* k;        // K 32-row blocks (mi::k_offset)
   const _Float16* v;        // V blocks, (r,h,i) at v + ((r/8)*G + h)*D*8 + i*8 + r%8
@@ -65,7 +75,8 @@ struct SplitArgs {
   // Flat split of up to kFusedPlan sequences: no plan kernel; every
   // workgroup computes the tile offsets into LDS from lengths / offsets, and
   // workgroup (0, 0) also stores them here (= tile_off) for the merge kernel.
-  // Null otherwise.
+  // Null otherwise.  With few tiles (kChunkTiles) the table counts chunks of
+  // whole sequences instead, and its last entry is stored as -1 - chunks.
   int32_t* tile_off_out;
   int batch;
   // Optional fused append (decode step, verify): rows [app0, app0 + app_n)
@@ -401,7 +412,8 @@ attn_split_kernel(SplitArgs a, X x) {
 
   constexpr bool flat = FLAT;  // the flat ragged split (a.tile_off)
   int64_t len = 0, row0 = 0, lim0 = 0, key_begin = 0, key_end = 0;
-  int64_t t_lo = 0, t_hi = 0;  // flat: this workgroup's tiles of the concatenation
+  int64_t t_lo = 0, t_hi = 0;  // flat: this workgroup's tiles (chunks) of the concatenation
+  int per_seq = 0;             // flat, by chunks of a sequence: tiles per chunk (else 0)
   // flat: the tile offsets, from the plan kernel's table or computed below
   int32_t* const ltoff = (int32_t*)(smem + GH * (NWH * ncols * (D + 4) + 2 * NWH * ncols));
   auto toff = [&](int i) -> int64_t {  // tile_off[i], i wave-uniform in [0, batch]
@@ -413,7 +425,7 @@ attn_split_kernel(SplitArgs a, X x) {
       // to kFusedPlan sequences, 64 per step, into LDS; workgroup (0, 0)
       // also stores them for the merge kernel.
       if (wv == 0) {
-        int32_t n[kFusedPlan / 64];
+        int32_t n[kFusedPlan / 64], per = 0;
 #pragma unroll
         for (int c = 0; c < kFusedPlan / 64; c++) {
           const int i = 64 * c + lane;
@@ -425,36 +437,51 @@ attn_split_kernel(SplitArgs a, X x) {
           }
         }
         const bool store = blockIdx.x == 0 && blockIdx.y == 0;
-        int32_t carry = 0;
+        // exclusive scan of n into LDS; returns the sum
+        auto scan = [&] {
+          int32_t carry = 0;
 #pragma unroll
-        for (int c = 0; c < kFusedPlan / 64; c++) {
-          int32_t inc = n[c];
+          for (int c = 0; c < kFusedPlan / 64; c++) {
+            int32_t inc = n[c];
 #pragma unroll
-          for (int d = 1; d < 64; d <<= 1) {
-            const int32_t y = __shfl_up(inc, d, 64);
-            if (lane >= d) inc += y;
+            for (int d = 1; d < 64; d <<= 1) {
+              const int32_t y = __shfl_up(inc, d, 64);
+              if (lane >= d) inc += y;
+            }
+            if (64 * c + lane < a.batch) ltoff[64 * c + lane] = carry + inc - n[c];
+            carry += __shfl(inc, 63, 64);
           }
-          const int i = 64 * c + lane;
-          if (i < a.batch) {
-            ltoff[i] = carry + inc - n[c];
-            if (store) a.tile_off_out[i] = carry + inc - n[c];
-          }
-          carry += __shfl(inc, 63, 64);
+          return carry;
+        };
+        int32_t carry = scan();
+        const int32_t spare = (int32_t)gridDim.x - a.batch;
+        if (spare > 0 && carry <= kChunkTiles * spare) {
+          per = max(1, (carry + spare - 1) / spare);
+#pragma unroll
+          for (int c = 0; c < kFusedPlan / 64; c++) n[c] = (n[c] + per - 1) / per;
+          carry = scan();
+        }
+        if (store) {
+#pragma unroll
+          for (int c = 0; c < kFusedPlan / 64; c++)  // the wave's own LDS entries
+            if (64 * c + lane < a.batch) a.tile_off_out[64 * c + lane] = ltoff[64 * c + lane];
         }
         if (lane == 0) {
           ltoff[a.batch] = carry;
-          if (store) a.tile_off_out[a.batch] = carry;
+          ltoff[kFusedPlan + 1] = per;
+          if (store) a.tile_off_out[a.batch] = per ? -1 - carry : carry;
         }
       }
       __syncthreads();
     }
     // min(gridDim.x, T) workgroups take the tiles, each at least one
     // (uniform values: kept in scalar registers)
+    if (a.tile_off_out) per_seq = __builtin_amdgcn_readfirstlane(ltoff[kFusedPlan + 1]);
     const int64_t total = toff(a.batch);
-    const int64_t nw = min((int64_t)gridDim.x, total);
+    const int64_t nw = per_seq ? total : min((int64_t)gridDim.x, total);
     if (chunk_idx >= nw) return;  // uniform
-    t_lo = (int64_t)chunk_idx * total / nw;
-    t_hi = (int64_t)(chunk_idx + 1) * total / nw;
+    t_lo = per_seq ? chunk_idx : (int64_t)chunk_idx * total / nw;
+    t_hi = per_seq ? chunk_idx + 1 : (int64_t)(chunk_idx + 1) * total / nw;
     // the sequence holding tile t_lo: the last s with tile_off[s] <= t_lo
     int lo = 0, hi = a.batch - 1;
     while (lo < hi) {
@@ -592,8 +619,9 @@ attn_split_kernel(SplitArgs a, X x) {
     len = __builtin_amdgcn_readfirstlane(a.lengths[s]);
     row0 = __builtin_amdgcn_readfirstlane(a.offsets[s]);
     lim0 = len;
-    key_begin = 32 * (max(t_lo, ps) - ps);
-    key_end = min(32 * (min(t_hi, pe) - ps), len);
+    const int64_t unit = 32 * (per_seq ? per_seq : 1);  // keys of an entry of the table
+    key_begin = unit * (max(t_lo, ps) - ps);
+    key_end = min(unit * (min(t_hi, pe) - ps), len);
     pslot = (int64_t)chunk_idx + s;
   }
 
@@ -1062,7 +1090,6 @@ struct CombineArgs {
   const int32_t* tile_off;  // flat ragged split (SplitArgs::tile_off), else null
   int nwg, batch;           // flat: the split launch's gridDim.x; sequences
   int64_t nslots;           // partial slots per KV head (SplitArgs::nslots)
-  bool wide;                // partials of the wide pass: a token's are those its row block wrote
 };
 
 // Chunk merge.  One workgroup per (column, KV head x slice of S values of
@@ -1082,7 +1109,8 @@ extern "C" __device__ float __ockl_wfred_add_f32(float);
 // S = kCombineSlice values of d per workgroup: 16 for up to 16 columns
 // (decode), 32 for the 32-column verify (measured: decode step 18.9 / 19.2 /
 // 19.3 us with S = 16 / 32 / 8, verify 33.1 / 32.7 / 34.6 us).
-template <int kCombineSlice>
+// WIDE: partials of the wide pass, where a token's are those of its row block.
+template <int kCombineSlice, bool WIDE = false>
 __global__ void __launch_bounds__(256)
 attn_combine_kernel(CombineArgs a) {
   constexpr int kCombineGroups = 256 / kCombineSlice;  // chunk groups of a workgroup
@@ -1104,7 +1132,7 @@ attn_combine_kernel(CombineArgs a) {
     bad = len < 0 || len > a.kv_len || off < 0 || (off & 31);
     if (bad) len = 0;
   }
-  if (a.wide) len = mi::wide_end((int)len - a.nq, a.nq, c >> 7);
+  if constexpr (WIDE) len = mi::wide_end((int)len - a.nq, a.nq, c >> 7);
   const int nch = (int)((len + a.chunk - 1) / a.chunk);
   const int64_t base = (int64_t)s * a.max_chunks;  // first partial slot of s
   const float* ml = a.part_ml + ((kvh * a.nslots + base) * ncols + c) * 2;  // chunk ch at ml[ch * mstride]
@@ -1194,7 +1222,10 @@ attn_combine_flat_kernel(CombineArgs a) {
   const int64_t total = a.tile_off[a.batch];
   const int64_t ps = a.tile_off[s], pe = a.tile_off[s + 1];
   int64_t first = 0, nch = 0;
-  if (pe > ps) {
+  if (total < 0) {  // by chunks of a sequence
+    first = ps;
+    nch = (s + 1 < a.batch ? pe : -1 - total) - ps;
+  } else if (pe > ps) {
     const int64_t nw = min((int64_t)a.nwg, total);
     first = ((ps + 1) * nw + total - 1) / total - 1;
     nch = (pe * nw + total - 1) / total - 1 - first + 1;
@@ -1203,30 +1234,38 @@ attn_combine_flat_kernel(CombineArgs a) {
   const float* ml = a.part_ml + slot0 * 2;
   const float* po = a.part_o + slot0 * D + d;
   float M = kNegBig, L = 0.f, o = 0.f;
-  constexpr int kB = 8;  // partials loaded per batch, all before their use
-  for (int64_t c0 = 0; c0 < nch; c0 += kB) {
-    float mb[kB], lb[kB], ob[kB];
+  // kB partials are loaded per batch, all before their use: 8, or 16 where a
+  // sequence has more (a small batch: 8 sequences of 1550 rows 25.7 -> 16.0 us
+  // per call with the chunks of one sequence; 16 for all cost 200 sequences of
+  // two partials 45 -> 50 us).
+  auto merge = [&](auto batch) {
+    constexpr int kB = decltype(batch)::value;
+    for (int64_t c0 = 0; c0 < nch; c0 += kB) {
+      float mb[kB], lb[kB], ob[kB];
 #pragma unroll
-    for (int k = 0; k < kB; k++) {
-      const bool in = c0 + k < nch;
-      mb[k] = in ? ml[(c0 + k) * ncols * 2] : kNegBig;
-      lb[k] = in ? ml[(c0 + k) * ncols * 2 + 1] : 0.f;
-      ob[k] = in ? po[(c0 + k) * ncols * D] : 0.f;
+      for (int k = 0; k < kB; k++) {
+        const bool in = c0 + k < nch;
+        mb[k] = in ? ml[(c0 + k) * ncols * 2] : kNegBig;
+        lb[k] = in ? ml[(c0 + k) * ncols * 2 + 1] : 0.f;
+        ob[k] = in ? po[(c0 + k) * ncols * D] : 0.f;
+      }
+      float mx = M;
+#pragma unroll
+      for (int k = 0; k < kB; k++) mx = fmaxf(mx, mb[k]);
+      const float sc = exp2f(M - mx);  // rescale what has been summed
+      L *= sc;
+      o *= sc;
+      M = mx;
+#pragma unroll
+      for (int k = 0; k < kB; k++) {
+        const float wgt = exp2f(mb[k] - M);
+        L += lb[k] * wgt;
+        o += ob[k] * wgt;
+      }
     }
-    float mx = M;
-#pragma unroll
-    for (int k = 0; k < kB; k++) mx = fmaxf(mx, mb[k]);
-    const float sc = exp2f(M - mx);  // rescale what has been summed
-    L *= sc;
-    o *= sc;
-    M = mx;
-#pragma unroll
-    for (int k = 0; k < kB; k++) {
-      const float wgt = exp2f(mb[k] - M);
-      L += lb[k] * wgt;
-      o += ob[k] * wgt;
-    }
-  }
+  };
+  if (nch <= 8) merge(std::integral_constant<int, 8>{});
+  else merge(std::integral_constant<int, 16>{});
   float r = (L > 0.f) ? o / L : 0.f;
   if (bad) r = __builtin_nanf("");
   const int hq = kvh * 8 + c;
@@ -1295,7 +1334,7 @@ mi_status launch_split(const SplitArgs& a, int64_t batch, hipStream_t stream, co
   const int ncols = a.nq * 8;
   size_t lds = (size_t)GH * (NWH * ncols * (D + 4) + 2 * NWH * ncols) * sizeof(float);
   if constexpr (is_proj<X>::value) lds += (size_t)GH * 8 * (D + 8) * sizeof(_Float16);
-  if constexpr (FLAT) lds += (size_t)(kFusedPlan + 1) * sizeof(int32_t);
+  if constexpr (FLAT) lds += (size_t)(kFusedPlan + 2) * sizeof(int32_t);
   static std::atomic<uint64_t> lds_set{0};
   // (below 160 KiB: the kernel also holds a few bytes of static LDS)
   MI_TRY(mi::set_lds_limit((const void*)attn_split_kernel<NWH, NCB, GH, X, FLAT>, 159 * 1024, lds_set));
@@ -1492,7 +1531,6 @@ mi_status run_split(const _Float16* k, const _Float16* v, const int32_t* offsets
   c.nslots = a.nslots;
   c.nwg = nwg;
   c.batch = (int)batch;
-  c.wide = false;
   if (lengths) {
     MI_HIP(mi::launch("attn_combine", attn_combine_flat_kernel, dim3(8, G, (unsigned)batch),
                       dim3(D), 0, stream, c));
@@ -1622,7 +1660,6 @@ mi_status wide_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float1
   c.max_chunks = nchunks;
   c.batch = 1;
   c.nslots = nchunks;
-  c.wide = true;
   // 16-byte lanes per column fill the CUs from 64 tokens on; for fewer with
   // many chunks (16 tokens at 65536 rows: 114) a workgroup per column and
   // 32-value slice does.  The rows form moves 8-byte pieces of gate and out.
@@ -1630,8 +1667,8 @@ mi_status wide_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float1
     MI_HIP(mi::launch("attn_combine", attn_combine_rows_kernel, dim3(n * 2, G), dim3(256), 0,
                       stream, c));
   else
-    MI_HIP(mi::launch("attn_combine", attn_combine_kernel<32>, dim3(n * 8, G * (D / 32), 1),
-                      dim3(256), 0, stream, c));
+    MI_HIP(mi::launch("attn_combine", attn_combine_kernel<32, true>,
+                      dim3(n * 8, G * (D / 32), 1), dim3(256), 0, stream, c));
   return MI_OK;
 }
 
@@ -1787,6 +1824,14 @@ mi_status attend_cache(mi_kv* kv, int32_t layer, const _Float16* q, const _Float
 bool attend_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
                    _Float16* out, int64_t past, int32_t n, hipStream_t stream, mi_status* st) {
   if (!takes_direct(past, n, gate, out)) return false;
+  // The workspace an eager split-K call of this size leaves for later captured
+  // calls, although this form needs none.
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  void* ws;
+  if (past >= 2048 && past >= 2 * (int64_t)n && hipStreamIsCapturing(stream, &cs) == hipSuccess &&
+      cs == hipStreamCaptureStatusNone &&
+      (*st = mi::kv_workspace(kv, wide_launch(kv->G, past, n).ws_bytes, stream, &ws)) != MI_OK)
+    return true;
   *st = run_direct(kv, layer, q, gate, out, past, n, stream, nullptr, nullptr, nullptr);
   return true;
 }

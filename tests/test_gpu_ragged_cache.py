@@ -47,6 +47,29 @@ def test_ragged_matches_oracle(lengths):
     assert np.all(o[lengths == 0] == 0)
 
 
+@pytest.mark.parametrize("lengths", [
+    [16 * 127 * 32], [16 * 127 * 32 + 1],  # the last length dealt by chunks, the first by tiles
+    [0, 40, 0, 0, 700, 1, 0],              # chunks skip empty sequences
+    [0, 0, 0],                             # nothing to attend
+    [33] * 127, [33] * 128,                # one spare workgroup, none
+    [16 * 32 + 5] * 120 + [0, 9]])         # chunks of 16 tiles and the rest of a sequence
+def test_ragged_chunks_of_one_sequence(lengths):
+    """Batches of few tiles go by chunks of a sequence (2 KV heads: 128
+    workgroups a head), each against the oracle."""
+    announce(f"ragged chunks batch={len(lengths)} rows={sum(lengths)}")
+    rng = np.random.default_rng(sum(lengths) + len(lengths))
+    lengths = np.array(lengths, np.int32)
+    offsets, k, v = ragged_buffers(rng, lengths)
+    b = len(lengths)
+    q, g = f16(rng, b, H, D), f16(rng, b, H, D)
+    kb, vb = kv_pack(dev(k), dev(v), G)
+    out = attn_decode_ragged(kb, vb, torch.from_numpy(offsets).cuda(),
+                             torch.from_numpy(lengths).cuda(), dev(q), max(1, int(lengths.max())),
+                             gate=dev(g))
+    assert_close(out, O.decode_ragged(q, k, v, offsets, lengths, gate=g), f"ragged chunks b={b}")
+    assert np.all(host(out)[lengths == 0] == 0)
+
+
 def test_ragged_c3_shape():
     """BASELINE config C3: 64 sequences, lengths U[1024, 32768] (seed 3);
     8 sequences are checked against the oracle, all 64 against the GPU
