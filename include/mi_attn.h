@@ -194,11 +194,12 @@ mi_status mi_attn_prefill(mi_kv* kv, int32_t layer, const mi_f16* q,
 
 /* K-token verify for speculative decoding: same contract as mi_attn_prefill
  * (append at past_pos, query i attends [0, past_pos + i]) for small n, run
- * split-K over the cache: up to 4 tokens in the decode kernel's form, more
- * in one pass of the prefill's MFMA tiles over key chunks that reads each
- * K/V tile once per 16 tokens (MI_ATTN_VERIFY_WIDE=0 runs them as 4-token
- * groups instead), then a merge; short contexts (1024 + 80 (n - 1) rows for up
- * to 16 tokens) in one launch.  Rollback afterwards is
+ * split-K over the cache: up to 4 tokens in the decode kernel's form, 5 to 16
+ * as groups of four in one such launch up to 20480 rows, else in one pass of
+ * the prefill's MFMA tiles over key chunks that reads each K/V tile once per 16
+ * tokens (MI_ATTN_VERIFY_WIDE=0 runs one launch pair per four tokens instead),
+ * then a merge; short contexts (1024 + 80 (n - 1) rows for up to 4 tokens, 1400
+ * + 21 n for up to 16) in one launch.  Rollback afterwards is
  * mi_kv_set_pos.  k = v = NULL as for mi_attn_prefill. */
 mi_status mi_attn_verify(mi_kv* kv, int32_t layer, const mi_f16* q,
                          const mi_f16* k, const mi_f16* v, const mi_f16* gate,

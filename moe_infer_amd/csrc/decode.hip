@@ -65,6 +65,7 @@ struct SplitArgs {
   float* part_ml;           // [G][nslots][ncols][2]  (flat ragged: slot = workgroup + s)
   int64_t nslots;
   int G, H, nq, chunk, max_chunks;
+  int ntok;                 // groups: query tokens in all
   float scale_log2e;
   // Flat ragged split: tile_off[s] = 32-key tiles of sequences 0..s-1
   // (invalid descriptors count 0), tile_off[batch] = all tiles T; workgroup
@@ -393,7 +394,11 @@ __device__ void merge_tail(const SplitArgs& a) {
 // With X = Proj (decode step from projections, one token, NCB = 1) the
 // kernel also norms and rotates Q per wave, and the workgroup holding row
 // app0 norms, rotates and appends K and appends V.
-template <int NWH, int NCB, int GH, typename X, bool FLAT>
+// With GROUPS the grid's z counts groups of nq query tokens of one sequence
+// (token tok0 = nq z on, the last group perhaps fewer): every group reads the
+// whole range, and workgroups of a chunk that holds new rows append the same
+// bytes, each before its own reads.
+template <int NWH, int NCB, int GH, typename X, bool FLAT, bool GROUPS = false>
 __global__ void __launch_bounds__(NWH * GH * 64)
 attn_split_kernel(SplitArgs a, X x) {
   constexpr bool kProj = is_proj<X>::value;
@@ -500,6 +505,7 @@ attn_split_kernel(SplitArgs a, X x) {
     len = a.kv_len;
     row0 = 0;
     lim0 = a.lim0;
+    if constexpr (GROUPS) lim0 += s * a.nq;
   }
   if constexpr (!flat) {
     key_begin = (int64_t)chunk_idx * a.chunk;
@@ -663,7 +669,7 @@ attn_split_kernel(SplitArgs a, X x) {
   for (int cb = 0; cb < NCB; cb++) {
     const int c = cb * 16 + j;
     const int tok = c >> 3;
-    if (c < ncols) {
+    if (c < ncols && (!GROUPS || s * a.nq + tok < a.ntok)) {
       const _Float16* qp =
           a.q + (((int64_t)s * a.nq + tok) * a.H + kvh * 8 + (c & 7)) * D + 8 * g;
 #pragma unroll
@@ -1090,6 +1096,7 @@ struct CombineArgs {
   const int32_t* tile_off;  // flat ragged split (SplitArgs::tile_off), else null
   int nwg, batch;           // flat: the split launch's gridDim.x; sequences
   int64_t nslots;           // partial slots per KV head (SplitArgs::nslots)
+  int ntok;                 // token groups: query tokens in all
 };
 
 // Chunk merge.  One workgroup per (column, KV head x slice of S values of
@@ -1109,8 +1116,10 @@ extern "C" __device__ float __ockl_wfred_add_f32(float);
 // S = kCombineSlice values of d per workgroup: 16 for up to 16 columns
 // (decode), 32 for the 32-column verify (measured: decode step 18.9 / 19.2 /
 // 19.3 us with S = 16 / 32 / 8, verify 33.1 / 32.7 / 34.6 us).
-// WIDE: partials of the wide pass, where a token's are those of its row block.
-template <int kCombineSlice, bool WIDE = false>
+// KIND: the launch's sequences (or the one) with their own lengths; the wide
+// pass, where a token's partials are those of its row block; or token groups.
+enum CombineKind { kSequences, kWide, kGroups };
+template <int kCombineSlice, CombineKind KIND = kSequences>
 __global__ void __launch_bounds__(256)
 attn_combine_kernel(CombineArgs a) {
   constexpr int kCombineGroups = 256 / kCombineSlice;  // chunk groups of a workgroup
@@ -1124,6 +1133,7 @@ attn_combine_kernel(CombineArgs a) {
   const int t = threadIdx.x;
   const int wv = t >> 6;
   const int ncols = a.nq * 8;
+  if (KIND == kGroups && s * a.nq + (c >> 3) >= a.ntok) return;  // whole workgroups
   int64_t len = a.kv_len;
   bool bad = false;
   if (a.lengths) {
@@ -1132,7 +1142,7 @@ attn_combine_kernel(CombineArgs a) {
     bad = len < 0 || len > a.kv_len || off < 0 || (off & 31);
     if (bad) len = 0;
   }
-  if constexpr (WIDE) len = mi::wide_end((int)len - a.nq, a.nq, c >> 7);
+  if constexpr (KIND == kWide) len = mi::wide_end((int)len - a.nq, a.nq, c >> 7);
   const int nch = (int)((len + a.chunk - 1) / a.chunk);
   const int64_t base = (int64_t)s * a.max_chunks;  // first partial slot of s
   const float* ml = a.part_ml + ((kvh * a.nslots + base) * ncols + c) * 2;  // chunk ch at ml[ch * mstride]
@@ -1329,7 +1339,7 @@ SplitPlan plan_split(int64_t max_len, int64_t batch, int G, int nq) {
   return mi::plan_split(max_len, batch, G, nq, split_knobs());
 }
 
-template <int NWH, int NCB, int GH, typename X = NoProj, bool FLAT = false>
+template <int NWH, int NCB, int GH, typename X = NoProj, bool FLAT = false, bool GROUPS = false>
 mi_status launch_split(const SplitArgs& a, int64_t batch, hipStream_t stream, const X& x = X()) {
   const int ncols = a.nq * 8;
   size_t lds = (size_t)GH * (NWH * ncols * (D + 4) + 2 * NWH * ncols) * sizeof(float);
@@ -1337,9 +1347,9 @@ mi_status launch_split(const SplitArgs& a, int64_t batch, hipStream_t stream, co
   if constexpr (FLAT) lds += (size_t)(kFusedPlan + 2) * sizeof(int32_t);
   static std::atomic<uint64_t> lds_set{0};
   // (below 160 KiB: the kernel also holds a few bytes of static LDS)
-  MI_TRY(mi::set_lds_limit((const void*)attn_split_kernel<NWH, NCB, GH, X, FLAT>, 159 * 1024, lds_set));
+  MI_TRY(mi::set_lds_limit((const void*)attn_split_kernel<NWH, NCB, GH, X, FLAT, GROUPS>, 159 * 1024, lds_set));
   dim3 grid(a.max_chunks, a.G / GH, (unsigned)batch);
-  MI_HIP(mi::launch("attn_split", attn_split_kernel<NWH, NCB, GH, X, FLAT>, grid,
+  MI_HIP(mi::launch("attn_split", attn_split_kernel<NWH, NCB, GH, X, FLAT, GROUPS>, grid,
                     dim3(NWH * GH * 64), lds, stream, a, x));
   return MI_OK;
 }
@@ -1412,7 +1422,8 @@ size_t ragged_workspace_bytes(int64_t batch, int G, int nwg) {
   return split_workspace_bytes(1, G, nwg + (int)batch, 1) + (size_t)(batch + 1) * sizeof(int32_t);
 }
 
-// Runs split + combine for nq <= 4 query tokens per sequence.
+// Runs split + combine for nq <= 4 query tokens per sequence, or with ntok > 0
+// for ntok tokens of one sequence in `batch` groups of nq = 4.
 struct AppendRows {
   const _Float16* k = nullptr;
   const _Float16* v = nullptr;
@@ -1426,7 +1437,7 @@ mi_status run_split(const _Float16* k, const _Float16* v, const int32_t* offsets
                     const _Float16* q, const _Float16* gate, _Float16* out,
                     void* ws, size_t ws_bytes, hipStream_t stream,
                     const AppendRows& app = AppendRows(), const ProjArgs* proj = nullptr,
-                    const mi_kv* kv = nullptr) {
+                    const mi_kv* kv = nullptr, int ntok = 0) {
   const SplitPlan plan = plan_split(max_len, batch, G, nq);
   SplitArgs a;
   a.mcnt = nullptr;
@@ -1440,6 +1451,7 @@ mi_status run_split(const _Float16* k, const _Float16* v, const int32_t* offsets
   a.G = G;
   a.H = H;
   a.nq = nq;
+  a.ntok = ntok;
   a.chunk = plan.chunk;
   a.max_chunks = plan.max_chunks;
   a.scale_log2e = mi::kLog2e / sqrtf((float)D);
@@ -1505,7 +1517,9 @@ mi_status run_split(const _Float16* k, const _Float16* v, const int32_t* offsets
   } else if (lengths) {
     st = plan.gh == 2 ? launch_split<4, 1, 2, NoProj, true>(a, 1, stream)
                       : launch_split<8, 1, 1, NoProj, true>(a, 1, stream);
-  } else if (plan.ncb == 2)
+  } else if (ntok)
+    st = launch_split<4, 2, 1, NoProj, false, true>(a, batch, stream);
+  else if (plan.ncb == 2)
     st = launch_split<4, 2, 1>(a, batch, stream);
   else if (plan.gh == 2)
     st = launch_split<4, 1, 2>(a, batch, stream);
@@ -1531,12 +1545,16 @@ mi_status run_split(const _Float16* k, const _Float16* v, const int32_t* offsets
   c.nslots = a.nslots;
   c.nwg = nwg;
   c.batch = (int)batch;
+  c.ntok = ntok;
   if (lengths) {
     MI_HIP(mi::launch("attn_combine", attn_combine_flat_kernel, dim3(8, G, (unsigned)batch),
                       dim3(D), 0, stream, c));
     return MI_OK;
   }
-  if (nq > 2) {
+  if (ntok) {
+    MI_HIP(mi::launch("attn_combine", attn_combine_kernel<32, kGroups>,
+                      dim3(nq * 8, G * (D / 32), (unsigned)batch), dim3(256), 0, stream, c));
+  } else if (nq > 2) {
     MI_HIP(mi::launch("attn_combine", attn_combine_kernel<32>, dim3(nq * 8, G * (D / 32), (unsigned)batch),
                       dim3(256), 0, stream, c));
   } else {
@@ -1667,7 +1685,7 @@ mi_status wide_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float1
     MI_HIP(mi::launch("attn_combine", attn_combine_rows_kernel, dim3(n * 2, G), dim3(256), 0,
                       stream, c));
   else
-    MI_HIP(mi::launch("attn_combine", attn_combine_kernel<32, true>,
+    MI_HIP(mi::launch("attn_combine", attn_combine_kernel<32, kWide>,
                       dim3(n * 8, G * (D / 32), 1), dim3(256), 0, stream, c));
   return MI_OK;
 }
@@ -1738,9 +1756,28 @@ mi_status cache_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float
                        const _Float16* k_new = nullptr, const _Float16* v_new = nullptr) {
   const bool direct = takes_direct(past_pos, n, gate, out);
   if (n > 4 && verify_wide_enabled()) {
-    if (!direct) return wide_attend(kv, layer, q, gate, out, past_pos, n, stream, k_new, v_new);
-    void* ws;  // as below
-    MI_TRY(mi::kv_workspace(kv, wide_launch(kv->G, past_pos, n).ws_bytes, stream, &ws));
+    const bool groups = !direct && mi::verify_groups(past_pos, n);
+    if (!direct && !groups)
+      return wide_attend(kv, layer, q, gate, out, past_pos, n, stream, k_new, v_new);
+    // (the wide form's workspace too: a later captured call may count on what
+    // an eager call of this size leaves)
+    const int ng = (n + 3) / 4;
+    size_t need = wide_launch(kv->G, past_pos, n).ws_bytes;
+    if (groups)
+      need = std::max(need, split_workspace_bytes(
+                                ng, kv->G, plan_split(past_pos + n, ng, kv->G, 4).max_chunks, 4));
+    void* ws;
+    MI_TRY(mi::kv_workspace(kv, need, stream, &ws));
+    if (groups) {
+      AppendRows app;
+      app.k = k_new;
+      app.v = v_new;
+      app.row0 = past_pos;
+      app.n = k_new ? n : 0;
+      return run_split(kv->k[layer], kv->v[layer], nullptr, nullptr, past_pos + n, past_pos + 1,
+                       past_pos + n, ng, kv->H, kv->G, 4, q, gate, out, ws, kv->ws_bytes, stream,
+                       app, nullptr, kv, n);
+    }
     return run_direct(kv, layer, q, gate, out, past_pos, n, stream, k_new, v_new, nullptr);
   }
   const int64_t lim0 = past_pos + 1;

@@ -227,8 +227,9 @@ inline WidePlan wide_plan(int G, int64_t past, int n) {
 // about 10 us whatever the length.
 // Up to 16 tokens, measured from HBM (us, one launch against the split forms):
 // 1 token at 517 rows 7.1 / 10.9, at 1000 9.4 / 10.8, at 1100 13.2 / 10.9; 4
-// tokens at 1000 9.7 / 15.5, at 1500 16.1 / 14.4; 8 at 1500 15.5 / 19.7, at
-// 2000 19.7 / 17.5; 16 at 2000 19.5 / 24.4, at 3000 27.0 / 25.1.
+// tokens at 1000 9.7 / 15.5, at 1500 16.1 / 14.4; 8 at 1500 15.5 / 15.9; 12 at
+// 1500 15.1 / 16.8, at 2000 19.3 / 16.9; 16 at 1500 15.1 / 18.0, at 2000 19.5 /
+// 18.2.
 // More tokens, without their append (against the prefill grid / the split-K
 // pass): 64 after 1000 rows 10.4 / 35.3 / 24.2, 128 after 3000 27.8 / 82.2 /
 // 28.9, 400 after 1000 30.3 / 45.1 / 32.8, 777 from none 25.5 / 30.9 / 42.3;
@@ -236,9 +237,20 @@ inline WidePlan wide_plan(int G, int64_t past, int n) {
 // / 36.6, 17 after 5000 33.6 / 119.7 / 25.0.
 inline bool direct_rows(int64_t past, int32_t n) {
   const int64_t rows = past + n;
-  if (n <= 16) return rows <= 1024 + 80 * (n - 1);
+  if (n <= 4) return rows <= 1024 + 80 * (n - 1);
+  if (n <= 16) return rows <= 1400 + 21 * n;
   return rows <= 3200 && n * (past + n / 2) <= 480000;
 }
+
+// Whether a verify of 5 to 16 tokens outside that runs as groups of four tokens
+// in one split launch (and one merge, the append inside) rather than in the
+// wide pass (append, pass, merge).  Every group reads the whole cache, but from
+// L2 and the last-level cache after the first, and a workgroup of the wide pass
+// has 8 us of Q and first tile and 6 us of epilogue.  Measured from HBM (us,
+// groups / wide): 8 tokens after 2300 rows 16.1 / 20.7, after 9001 18.8 / 26.0,
+// after 24000 27.6 / 28.2; 12 after 9001 19.8 / 30.9; 9 after 24000 31.0 / 29.7;
+// 16 after 16000 26.0 / 33.4, after 32000 40.2 / 38.1, after 65536 100 / 49.
+inline bool verify_groups(int64_t past, int32_t n) { return n <= 16 && past + n <= 20480; }
 
 // Whether a prefill outside that takes the split-K pass and its merge rather
 // than the prefill grid (one workgroup per 128 queries and head): the grid is

@@ -52,7 +52,10 @@ def test_step(past):
 
 
 @pytest.mark.parametrize("past,n", [(0, 2), (31, 3), (500, 4), (1260, 4), (1261, 4), (97, 5),
-                                    (2208, 16), (2209, 16), (300, 40)])
+                                    (1720, 16), (300, 40),
+                                    # groups of four tokens in one split launch, then the wide pass
+                                    (1721, 16), (1501, 5), (1800, 6), (4000, 9), (3001, 7), (20475, 5),
+                                    (20476, 5)])
 def test_verify(past, n):
     out, ref = causal_case(past, n, attn_verify)
     assert_close(out, ref, f"verify past={past} n={n}")
