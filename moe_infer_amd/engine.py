@@ -89,11 +89,11 @@ class EngineSnapshot:
     mtp_pos: int
 
 
-# Largest token count forward_batched sends to mi_attn_verify (split-K over
-# the cache: the decode kernel's form up to 4 tokens, the prefill tiles'
-# split-K form above), the speculative-verify case; more tokens go to
-# mi_attn_prefill, which itself splits over the past when the past is long
-# next to them.
+# Largest token count forward_batched sends to mi_attn_verify (the decode
+# kernel's forms, above 20480 rows and 4 tokens the prefill tiles' split-K
+# form), the speculative-verify case; more tokens go to mi_attn_prefill, which
+# itself runs short prompts in one launch and splits over the past when the
+# past is long next to them.
 VERIFY_MAX_TOKENS = 16
 
 
