@@ -195,6 +195,13 @@ MI_HD inline bool wide_item(int past, int n, int chunk, int idx, int& rb, int& c
   return true;
 }
 
+// Whether its workgroups go to the XCDs in runs that share K/V (a chunk's row
+// blocks) rather than one by one: once the past outgrows the L2s and its bytes
+// outweigh the blocks' work.  The times are at the mapping in the kernel.
+inline bool wide_runs(int64_t past, int32_t n) {
+  return n > 16 && past >= 12288 && past >= 64 * (int64_t)n;
+}
+
 // Its chunking: whole 64-key tiles, at most kMaxSplitChunks chunks (the merge
 // kernels' limit), and the smallest chunk whose workgroups all run at once (256
 // CUs): one more than that waits for a whole chunk.  Measured after 1000 rows,

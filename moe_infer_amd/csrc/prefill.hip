@@ -70,6 +70,8 @@ struct PrefillArgs {
 struct VerifyArgs {
   int64_t chunk;
   int nchunks, ncols;
+  int items;  // mi::wide_items: workgroups per KV head
+  int run;    // items of an XCD's run, or 0
   int64_t nslots;
   float* part_o;
   float* part_ml;
@@ -624,7 +626,10 @@ mi_status verify_wide_split(const mi_kv* kv, int32_t layer, const _Float16* q, i
   vx.nslots = nchunks;
   vx.part_o = part_o;
   vx.part_ml = part_ml;
-  return launch_verify_wide(a, vx, wide_items((int)past, n, (int)chunk) * kv->G, stream);
+  vx.items = wide_items((int)past, n, (int)chunk);
+  const int wgs = vx.items * kv->G;
+  vx.run = wide_runs(past, n) ? (wgs + 7) / 8 : 0;
+  return launch_verify_wide(a, vx, vx.run ? vx.run * 8 : wgs, stream);
 }
 
 }  // namespace mi
