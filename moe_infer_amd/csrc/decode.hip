@@ -869,7 +869,16 @@ struct DirectArgs {
 };
 
 constexpr int kDirectWaves = 4;
-template <int NDB, typename X>
+// TILE: a tile's weights are taken against the tile's own max, so that its
+// largest is exactly 1 in f16, and its sums are weighted in f32 - the precision
+// of the split forms, whose waves see one tile each at these lengths.  Against
+// the wave's running max, where only one of its tiles has such a weight, the
+// error against 64 bits was 3.5 % larger for a step at 517 rows, 6 % for a
+// verify of 8 at 1000, 9.5 % for one of 24 at 3100.  It costs 0.1 of 7.3 us at
+// 517 rows.  A prefill in slices of 16 value blocks (NDB = 16) goes without: the
+// prefill grid, which it stands for, is no closer (2.44e-4 either way for 333
+// tokens), and the weighting took 200 tokens after 600 rows from 13.7 to 14.5 us.
+template <int NDB, typename X, bool TILE>
 __global__ void __launch_bounds__(kDirectWaves * 64, 2)
 attn_direct_kernel(DirectArgs a, X x) {
   constexpr bool kProj = is_proj<X>::value;
@@ -996,7 +1005,7 @@ attn_direct_kernel(DirectArgs a, X x) {
     float mt = fmaxf(st[0][0], st[1][0]);
 #pragma unroll
     for (int e = 1; e < 4; e++) mt = fmaxf(mt, fmaxf(st[0][e], st[1][e]));
-    mt = mi::max_rows(mt) * c2;
+    mt = fmaxf(mi::max_rows(mt) * c2, kNegBig);  // (a column that sees no key: -inf)
     const float mnew = fmaxf(m, mt);
     if (__ballot(mnew != m)) {
       const float alpha = __builtin_amdgcn_exp2f(m - mnew);
@@ -1005,6 +1014,8 @@ attn_direct_kernel(DirectArgs a, X x) {
       for (int d = 0; d < NDB; d++) acc[d] *= alpha;
       m = mnew;
     }
+    const float mref = TILE ? mt : m;
+    const float wt = TILE ? __builtin_amdgcn_exp2f(mt - m) : 1.f;
     // The row sum adds the f16 weights the PV MFMA uses.
     float rs = 0.f;
     f16x8 pf;
@@ -1012,13 +1023,13 @@ attn_direct_kernel(DirectArgs a, X x) {
     for (int u = 0; u < 2; u++)
 #pragma unroll
       for (int e = 0; e < 4; e += 2) {
-        const f16x2 ph = {(_Float16)__builtin_amdgcn_exp2f(fmaf(st[u][e], c2, -m)),
-                          (_Float16)__builtin_amdgcn_exp2f(fmaf(st[u][e + 1], c2, -m))};
+        const f16x2 ph = {(_Float16)__builtin_amdgcn_exp2f(fmaf(st[u][e], c2, -mref)),
+                          (_Float16)__builtin_amdgcn_exp2f(fmaf(st[u][e + 1], c2, -mref))};
         rs = __builtin_amdgcn_fdot2(ph, f16x2{1.f16, 1.f16}, rs, false);
         pf[4 * u + e] = ph[0];
         pf[4 * u + e + 1] = ph[1];
       }
-    l += mi::sum_rows(rs);
+    l += mi::sum_rows(rs) * wt;
     if (32 * t + 32 > rows) {  // stale rows may hold anything, 0 * NaN is NaN
       const int valid = rows - (32 * t + 8 * g);
 #pragma unroll
@@ -1028,8 +1039,16 @@ attn_direct_kernel(DirectArgs a, X x) {
           if (e >= valid) vf[d][e] = (_Float16)0.f;
     }
 #pragma unroll
-    for (int d = 0; d < NDB; d++)
-      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[d], pf, acc[d], 0, 0, 0);
+    for (int d = 0; d < NDB; d++) {
+      if constexpr (TILE) {
+        acc[d] += wt * __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[d], pf, f32x4{0.f, 0.f, 0.f, 0.f},
+                                                              0, 0, 0);
+        // (all 16 products at once would spill)
+        if (NDB == 16 && d % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+      } else {
+        acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[d], pf, acc[d], 0, 0, 0);
+      }
+    }
     if (t + NWH < ntiles) load_v(t + NWH);
   }
 
@@ -1365,14 +1384,15 @@ mi_status launch_proj(const SplitArgs& a, const SplitPlan& plan, hipStream_t str
   return launch_split<8, 1, 1>(a, 1, stream, x);
 }
 
-template <int NDB, typename X = NoProj>
+template <int NDB, bool TILE = true, typename X = NoProj>
 mi_status launch_direct(const DirectArgs& a, hipStream_t stream, const X& x = X()) {
   size_t lds = (size_t)kDirectWaves * 16 * (NDB * 16 + 4 + 2) * sizeof(float);
   if constexpr (is_proj<X>::value) lds += (size_t)8 * (D + 8) * sizeof(_Float16);
   static std::atomic<uint64_t> lds_set{0};
-  MI_TRY(mi::set_lds_limit((const void*)attn_direct_kernel<NDB, X>, 80 * 1024, lds_set));
-  MI_HIP(mi::launch("attn_direct", attn_direct_kernel<NDB, X>, dim3((a.n + 1) / 2, a.G * (16 / NDB)),
-                    dim3(kDirectWaves * 64), lds, stream, a, x));
+  MI_TRY(mi::set_lds_limit((const void*)attn_direct_kernel<NDB, X, TILE>, 80 * 1024, lds_set));
+  MI_HIP(mi::launch("attn_direct", attn_direct_kernel<NDB, X, TILE>,
+                    dim3((a.n + 1) / 2, a.G * (16 / NDB)), dim3(kDirectWaves * 64), lds, stream, a,
+                    x));
   return MI_OK;
 }
 
@@ -1705,7 +1725,8 @@ constexpr int kDirectAppend = 16;
 
 mi_status run_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
                      _Float16* out, int64_t past, int32_t n, hipStream_t stream,
-                     const _Float16* k_new, const _Float16* v_new, const ProjArgs* proj) {
+                     const _Float16* k_new, const _Float16* v_new, const ProjArgs* proj,
+                     bool grid_precision = false) {
   if (k_new && n > kDirectAppend) {
     MI_TRY(mi::kv_append_rows(kv, layer, k_new, v_new, past, n, stream));
     k_new = v_new = nullptr;
@@ -1739,7 +1760,7 @@ mi_status run_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16
   const int wgs = (n + 1) / 2 * kv->G;
   if (wgs * 4 <= 256) return launch_direct<4>(a, stream);
   if (wgs * 2 <= 256) return launch_direct<8>(a, stream);
-  return launch_direct<16>(a, stream);
+  return grid_precision ? launch_direct<16, false>(a, stream) : launch_direct<16>(a, stream);
 }
 
 // Verify / decode over the cache: n query tokens at positions past_pos ..
@@ -1862,11 +1883,12 @@ bool attend_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* 
   // calls, although this form needs none.
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   void* ws;
-  if (past >= 2048 && past >= 2 * (int64_t)n && hipStreamIsCapturing(stream, &cs) == hipSuccess &&
+  const bool split = past >= 2048 && past >= 2 * (int64_t)n;  // else what the grid would run
+  if (split && hipStreamIsCapturing(stream, &cs) == hipSuccess &&
       cs == hipStreamCaptureStatusNone &&
       (*st = mi::kv_workspace(kv, wide_launch(kv->G, past, n).ws_bytes, stream, &ws)) != MI_OK)
     return true;
-  *st = run_direct(kv, layer, q, gate, out, past, n, stream, nullptr, nullptr, nullptr);
+  *st = run_direct(kv, layer, q, gate, out, past, n, stream, nullptr, nullptr, nullptr, !split);
   return true;
 }
 
