@@ -392,8 +392,13 @@ __device__ void merge_tail(const SplitArgs& a) {
 // With GROUPS the grid's z counts groups of nq query tokens of one sequence
 // (token tok0 = nq z on, the last group perhaps fewer): every group reads the
 // whole range, and workgroups of a chunk that holds new rows append the same
-// bytes, each before its own reads.
-template <int NWH, int NCB, int GH, typename X, bool FLAT, bool GROUPS = false>
+// bytes, each before its own reads.  TILE: a tile's weights against the tile's
+// own max (see attn_direct_kernel), where a wave has two tiles and the wide
+// pass, which also serves these sizes, has one: up to 16384 / G rows.  Without it
+// the error against 64 bits of 12 tokens after 6100 rows was 1.7 % above that
+// pass's; with it 12 after 9001 rows, where the wide pass is 5 % above, would
+// go from 19.5 to 20.0 us.
+template <int NWH, int NCB, int GH, typename X, bool FLAT, bool GROUPS = false, bool TILE = false>
 __global__ void __launch_bounds__(NWH * GH * 64)
 attn_split_kernel(SplitArgs a, X x) {
   constexpr bool kProj = is_proj<X>::value;
@@ -740,6 +745,8 @@ attn_split_kernel(SplitArgs a, X x) {
       mt = mi::max_rows(mt);
       const float mnew = fmaxf(m[cb], mt);
       const float alpha = exp2f(m[cb] - mnew);
+      const float mref = TILE ? mt : mnew;
+      const float wt = TILE ? exp2f(mt - mnew) : 1.f;
       float rs = 0.f;
       f16x8 pf;
 #pragma unroll
@@ -748,18 +755,22 @@ attn_split_kernel(SplitArgs a, X x) {
         for (int e = 0; e < 4; e++) {
           // The row sum adds the f16 weights the PV MFMA uses, so that the
           // normalised weights sum to one.
-          const _Float16 ph = (_Float16)exp2f(st[u][e] - mnew);
+          const _Float16 ph = (_Float16)exp2f(st[u][e] - mref);
           rs += (float)ph;
           pf[4 * u + e] = ph;
         }
       rs = mi::sum_rows(rs);
-      l[cb] = l[cb] * alpha + rs;
+      l[cb] = l[cb] * alpha + (TILE ? rs * wt : rs);
       m[cb] = mnew;
 #pragma unroll
       for (int dblk = 0; dblk < 16; dblk++) {
         acc[cb][dblk] *= alpha;
-        acc[cb][dblk] =
-            __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[dblk], pf, acc[cb][dblk], 0, 0, 0);
+        if constexpr (TILE)
+          acc[cb][dblk] += wt * __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                    vf[dblk], pf, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        else
+          acc[cb][dblk] =
+              __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[dblk], pf, acc[cb][dblk], 0, 0, 0);
       }
     }
   }
@@ -875,9 +886,10 @@ constexpr int kDirectWaves = 4;
 // the wave's running max, where only one of its tiles has such a weight, the
 // error against 64 bits was 3.5 % larger for a step at 517 rows, 6 % for a
 // verify of 8 at 1000, 9.5 % for one of 24 at 3100.  It costs 0.1 of 7.3 us at
-// 517 rows.  A prefill in slices of 16 value blocks (NDB = 16) goes without: the
-// prefill grid, which it stands for, is no closer (2.44e-4 either way for 333
-// tokens), and the weighting took 200 tokens after 600 rows from 13.7 to 14.5 us.
+// 517 rows.  A prefill in slices of 16 value blocks (NDB = 16) goes without: it
+// is closer than the prefill grid, which it stands for, as it is (2.44e-4 and
+// 2.50e-4 for 333 tokens, 2.63e-4 and 2.87e-4 for 200 after 600 rows), and the
+// weighting took the latter from 13.7 to 14.5 us.
 template <int NDB, typename X, bool TILE>
 __global__ void __launch_bounds__(kDirectWaves * 64, 2)
 attn_direct_kernel(DirectArgs a, X x) {
@@ -1353,7 +1365,8 @@ SplitPlan plan_split(int64_t max_len, int64_t batch, int G, int nq) {
   return mi::plan_split(max_len, batch, G, nq, split_knobs());
 }
 
-template <int NWH, int NCB, int GH, typename X = NoProj, bool FLAT = false, bool GROUPS = false>
+template <int NWH, int NCB, int GH, typename X = NoProj, bool FLAT = false, bool GROUPS = false,
+          bool TILE = false>
 mi_status launch_split(const SplitArgs& a, int64_t batch, hipStream_t stream, const X& x = X()) {
   const int ncols = a.nq * 8;
   size_t lds = (size_t)GH * (NWH * ncols * (D + 4) + 2 * NWH * ncols) * sizeof(float);
@@ -1361,9 +1374,10 @@ mi_status launch_split(const SplitArgs& a, int64_t batch, hipStream_t stream, co
   if constexpr (FLAT) lds += (size_t)(kFusedPlan + 2) * sizeof(int32_t);
   static std::atomic<uint64_t> lds_set{0};
   // (below 160 KiB: the kernel also holds a few bytes of static LDS)
-  MI_TRY(mi::set_lds_limit((const void*)attn_split_kernel<NWH, NCB, GH, X, FLAT, GROUPS>, 159 * 1024, lds_set));
+  MI_TRY(mi::set_lds_limit((const void*)attn_split_kernel<NWH, NCB, GH, X, FLAT, GROUPS, TILE>,
+                           159 * 1024, lds_set));
   dim3 grid(a.max_chunks, a.G / GH, (unsigned)batch);
-  MI_HIP(mi::launch("attn_split", attn_split_kernel<NWH, NCB, GH, X, FLAT, GROUPS>, grid,
+  MI_HIP(mi::launch("attn_split", attn_split_kernel<NWH, NCB, GH, X, FLAT, GROUPS, TILE>, grid,
                     dim3(NWH * GH * 64), lds, stream, a, x));
   return MI_OK;
 }
@@ -1533,7 +1547,9 @@ mi_status run_split(const _Float16* k, const _Float16* v, const int32_t* offsets
     st = plan.gh == 2 ? launch_split<4, 1, 2, NoProj, true>(a, 1, stream)
                       : launch_split<8, 1, 1, NoProj, true>(a, 1, stream);
   } else if (ntok)
-    st = launch_split<4, 2, 1, NoProj, false, true>(a, batch, stream);
+    st = a.chunk > 4 * 32 && max_len * G <= 16384
+             ? launch_split<4, 2, 1, NoProj, false, true, true>(a, batch, stream)
+             : launch_split<4, 2, 1, NoProj, false, true>(a, batch, stream);
   else if (plan.ncb == 2)
     st = launch_split<4, 2, 1>(a, batch, stream);
   else if (plan.gh == 2)

@@ -134,7 +134,8 @@ def test_same_as_the_split_forms(monkeypatch, n):
     assert_close(one, host(call()), f"direct against split n={n}", atol=2.0 ** -10)
 
 
-@pytest.mark.parametrize("past,n", [(516, 1), (1000, 1), (1000, 12), (3100, 24)])
+@pytest.mark.parametrize("past,n", [(516, 1), (1000, 1), (1000, 12), (3100, 24),
+                                    (4300, 16), (6100, 12)])  # token groups, two tiles a wave
 def test_weights_of_the_split_forms(monkeypatch, past, n):
     """Both forms take a tile's f16 weights against the tile's own max, so the
     weights are the same numbers but for a rounding of the exponent (2^-22 of a
