@@ -132,8 +132,10 @@ constexpr int kMaxSplitChunks = 1024;
 // The wide verify / split-K prefill (attn_verify_wide_kernel): one workgroup
 // per KV head, row block rb of 16 tokens and chunk c that holds keys the
 // block's tokens see, rows [0, end(rb)).  Whole chunks come first, then every
-// block's last chunk, the longest first where there are several of a length: a
-// workgroup's time is its keys, and the launch ends with its last one.
+// block's last chunk, the latest block first.  No index is left empty: an empty
+// one takes a place in the round-robin over the XCDs from a workgroup, which
+// then waits for another's whole chunk (with empty indices among the last
+// chunks, 672 tokens after 1260 rows took 56.7 us, without 41.5).
 MI_HD inline int wide_end(int past, int n, int rb) {
   return past + (n < 16 * rb + 16 ? n : 16 * rb + 16);
 }
@@ -151,26 +153,20 @@ MI_HD inline int wide_count(int past, int n, int chunk) {  // workgroups
   for (; wide_first(past, n, chunk, c) < nrb; c++) items += nrb - wide_first(past, n, chunk, c);
   return items;
 }
-// Grid indices wide_item takes: the last chunks may leave holes among theirs.
-MI_HD inline int wide_items(int past, int n, int chunk) {
-  const int nrb = (n + 15) / 16, per = chunk / 16;
-  return wide_count(past, n, chunk) + (nrb <= per ? 0 : (nrb + per - 1) / per * per - nrb);
-}
-// Item idx of [0, wide_items): its row block and chunk; false for none.  (One
-// block, a verify of up to 16 tokens: the divisions below would cost it 0.25 of
-// 27 us.)
-MI_HD inline bool wide_item(int past, int n, int chunk, int idx, int& rb, int& c) {
+// Item idx of [0, wide_count): its row block and chunk.  (One block, a verify of
+// up to 16 tokens: the divisions below would cost it 0.25 of 27 us.)
+MI_HD inline void wide_item(int past, int n, int chunk, int idx, int& rb, int& c) {
   if (n <= 16) {
     rb = 0;
     c = idx;
-    return true;
+    return;
   }
-  const int nrb = (n + 15) / 16, per = chunk / 16;
+  const int nrb = (n + 15) / 16;
   int cc = past / chunk;
   if (idx < cc * nrb) {
     c = idx / nrb;
     rb = nrb - 1 - (idx - c * nrb);
-    return true;
+    return;
   }
   idx -= cc * nrb;
   for (;; cc++) {
@@ -179,20 +175,12 @@ MI_HD inline bool wide_item(int past, int n, int chunk, int idx, int& rb, int& c
     if (idx < nrb - first) {
       c = cc;
       rb = nrb - 1 - idx;
-      return true;
+      return;
     }
     idx -= nrb - first;
   }
-  if (nrb <= per) {
-    rb = nrb - 1 - idx;
-  } else {  // several runs of `per` blocks: the same place of each run in turn
-    const int runs = (nrb + per - 1) / per;
-    const int place = per - 1 - idx / runs;
-    rb = idx % runs * per + (place + per - past / 16 % per) % per;
-  }
-  if (rb >= nrb) return false;
+  rb = nrb - 1 - idx;
   c = (wide_end(past, n, rb) - 1) / chunk;
-  return true;
 }
 
 // Whether its workgroups go to the XCDs in runs that share K/V (a chunk's row
@@ -262,10 +250,13 @@ inline bool verify_groups(int64_t past, int32_t n) { return n <= 16 && past + n 
 // Whether a prefill outside that takes the split-K pass and its merge rather
 // than the prefill grid (one workgroup per 128 queries and head): the grid is
 // short of workgroups and each walks the whole past.  Measured, split-K
-// against the grid (us): 512 tokens after 1000 rows 42.8 / 48.4, 640 after 600
-// 35.0 / 42.9, 1024 after 1024 53 / 62, 512 after 16384 152 / 377; it loses
-// with 1024 after 600 (57 / 53) and from none (36.6 / 37.0 at 1024 tokens, 54 /
-// 50 at 1500), and beyond 1024 tokens, which leave no CU idle.
+// against the grid (us): 512 tokens after 1024 rows 34.3 / 46.8, 600 after 600
+// 33.3 / 38.8, 640 after 480 32.7 / 38.8, 777 after 777 40.4 / 50.4, 850 after
+// 850 44.0 / 50.4, 960 after 960 47.8 / 54.0, 1024 after 1024 49.5 / 58.0, 512
+// after 16384 139 / 377.  Nowhere in 300 sizes of 100 to 1024 tokens did the
+// grid win; below the line the lead shrinks with the past (777 after 291 34.4 /
+// 38.1, 1024 from none 33.9 / 35.6), and with more tokens no CU is idle (1200
+// from none 39.2 / 39.1).
 inline bool prefill_split_rows(int64_t past, int32_t n) {
   return n <= 1024 && past >= (n <= 640 ? n / 2 : n);
 }

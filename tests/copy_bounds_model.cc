@@ -112,10 +112,12 @@ static long long wide_violations(long long past, int n, long long cap) {
   // the items name every (row block, chunk) with visible keys exactly once
   const int nrb = (n + 15) / 16;
   std::vector<char> named((size_t)nrb * wp.nchunks, 0);
-  const int items = mi::wide_items((int)past, n, (int)wp.chunk);
+  const int items = mi::wide_count((int)past, n, (int)wp.chunk);
+  // one round of the 256 CUs, where the row blocks alone do not exceed it
+  if (nrb * 2 <= 256 && items * 2 > 256) bad++;
   for (int i = 0; i < items; i++) {
       int rb, c;
-      if (!mi::wide_item((int)past, n, (int)wp.chunk, i, rb, c)) continue;
+      mi::wide_item((int)past, n, (int)wp.chunk, i, rb, c);
       if (rb < 0 || rb >= nrb || c < 0 || c >= wp.nchunks || named[(size_t)rb * wp.nchunks + c]++) {
         bad++;
         continue;
