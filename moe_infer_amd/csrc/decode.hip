@@ -1716,9 +1716,10 @@ mi_status wide_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float1
     MI_HIP(mi::launch("attn_combine", attn_combine_rows_kernel, dim3(n * 2, G), dim3(256), 0,
                       stream, c));
   else
-    // (one row block writes every chunk: the kernel without the block's end)
+    // (the kernel without the block's end where every block writes every chunk)
     MI_HIP(mi::launch("attn_combine",
-                      n <= 16 ? attn_combine_kernel<32> : attn_combine_kernel<32, kWide>,
+                      mi::wide_full(past_pos, n, chunk, nchunks) ? attn_combine_kernel<32>
+                                                                 : attn_combine_kernel<32, kWide>,
                       dim3(n * 8, G * (D / 32), 1), dim3(256), 0, stream, c));
   return MI_OK;
 }

@@ -131,10 +131,10 @@ constexpr int kMaxSplitChunks = 1024;
 
 // The wide verify / split-K prefill (attn_verify_wide_kernel): one workgroup
 // per KV head, row block rb of 16 tokens and chunk c that holds keys the
-// block's tokens see, rows [0, end(rb)).  Whole chunks come first, then every
-// block's last chunk, the latest block first.  No index is left empty: an empty
-// one takes a place in the round-robin over the XCDs from a workgroup, which
-// then waits for another's whole chunk (with empty indices among the last
+// block's tokens see, rows [0, end(rb)).  As items, whole chunks come first, then
+// every block's last chunk, the latest block first.  No item is empty: an empty
+// grid index takes a place in the round-robin over the XCDs from a workgroup,
+// which then waits for another's whole chunk (with empty ones among the last
 // chunks, 672 tokens after 1260 rows took 56.7 us, without 41.5).
 MI_HD inline int wide_end(int past, int n, int rb) {
   return past + (n < 16 * rb + 16 ? n : 16 * rb + 16);
@@ -153,14 +153,8 @@ MI_HD inline int wide_count(int past, int n, int chunk) {  // workgroups
   for (; wide_first(past, n, chunk, c) < nrb; c++) items += nrb - wide_first(past, n, chunk, c);
   return items;
 }
-// Item idx of [0, wide_count): its row block and chunk.  (One block, a verify of
-// up to 16 tokens: the divisions below would cost it 0.25 of 27 us.)
+// Item idx of [0, wide_count): its row block and chunk.
 MI_HD inline void wide_item(int past, int n, int chunk, int idx, int& rb, int& c) {
-  if (n <= 16) {
-    rb = 0;
-    c = idx;
-    return;
-  }
   const int nrb = (n + 15) / 16;
   int cc = past / chunk;
   if (idx < cc * nrb) {
@@ -183,11 +177,69 @@ MI_HD inline void wide_item(int past, int n, int chunk, int idx, int& rb, int& c
   c = (wide_end(past, n, rb) - 1) / chunk;
 }
 
-// Whether its workgroups go to the XCDs in runs that share K/V (a chunk's row
-// blocks) rather than one by one: once the past outgrows the L2s and its bytes
-// outweigh the blocks' work.  The times are at the mapping in the kernel.
-inline bool wide_runs(int64_t past, int32_t n) {
-  return n > 16 && past >= 12288 && past >= 64 * (int64_t)n;
+// How the workgroups are dealt to the XCDs (blockIdx % 8):
+//   pitch > 0  (row block, chunk, KV head), the head fastest; pitch = chunks *
+//              heads (a last chunk that a block lacks is left empty: only where
+//              all still run at once)
+//   run > 0    each XCD takes a run of `run` items in (head, chunk, row block)
+//              order, so that the blocks of a chunk, which read the same K/V,
+//              share its L2
+//   else       (item, KV head), the head fastest: the blocks of a chunk one
+//              after the other
+// Measured (us, by block / runs / by item, from HBM): 17 tokens after 3500 rows
+// 25.3 / 26.0 / 24.7, after 9000 25.3 / 27.8 / 26.6, after 20000 30.9 / 29.0 /
+// 32.5; 40 after 4500 29.6 / 32.1 / 27.5, after 12000 31.9 / 31.8 / 33.6, after
+// 32000 44.7 / 44.4 / 49.4; 49 after 4500 32.9 / 34.3 / 31.5, after 12000 35.1 /
+// 35.7 / 39.7, after 64000 79.1 / 80.2 / -; 64 after 64000 82.2 / 82.8 / 93.9; 128
+// after 8000 37.4 / 38.2 / 35.6, after 64000 136.3 / 136.2 / 139.2; 256 after 8000
+// 52.0 / 53.1 / 50.0; 17 after 65000, where the chunks are a multiple of 8, 52.0 /
+// 53.0 / -.  A single row block (a verify of up to 16 tokens) goes by
+// block: its look-up is a division, the others' would cost it 0.4 of 35 us.
+struct WideDeal {
+  int items;  // wide_count: workgroups per KV head
+  int pitch, run;
+  int grid;  // workgroups launched
+};
+// Every block has every chunk.
+inline bool wide_full(int64_t past, int n, int64_t chunk, int nchunks) {
+  return wide_end((int)past, n, 0) > (int64_t)(nchunks - 1) * chunk;
+}
+inline WideDeal wide_deal(int G, int64_t past, int n, int64_t chunk, int nchunks) {
+  WideDeal d;
+  d.items = wide_count((int)past, n, (int)chunk);
+  d.pitch = d.run = 0;
+  d.grid = d.items * G;
+  const int nrb = (n + 15) / 16;
+  const bool runs = nrb > 1 && past >= 12288 && past >= 64 * (int64_t)n;
+  const bool shared = nchunks * G % 8 == 0;  // by block: a chunk's blocks on one XCD
+  const bool by_block = nrb == 1 || (nrb == 4 && past >= 5000) ||
+                        (nrb < 4 && past >= 6400 && (!runs || (nrb == 2 && shared)));
+  if (by_block && (nrb == 1 || nrb * nchunks * G <= 256)) {
+    d.pitch = nchunks * G;
+    d.grid = nrb * d.pitch;
+  } else if (runs) {
+    d.run = (d.grid + 7) / 8;
+    d.grid = 8 * d.run;
+  }
+  return d;
+}
+// Workgroup `block`'s row block, chunk and KV head; false for none.
+MI_HD inline bool wide_place(const WideDeal& d, int G, int past, int n, int chunk, int block,
+                             int& rb, int& c, int& kvh) {
+  if (d.pitch) {
+    rb = block / d.pitch;
+    const int u = block - rb * d.pitch;
+    c = u / G;
+    kvh = u - c * G;
+    return c * chunk < wide_end(past, n, rb);
+  }
+  const int idx = d.run ? (block & 7) * d.run + (block >> 3) : block;
+  const int per = d.run ? d.items : G;
+  const int hi = idx / per, lo = idx - hi * per;
+  kvh = d.run ? hi : lo;
+  if (kvh >= G) return false;
+  wide_item(past, n, chunk, d.run ? lo : hi, rb, c);
+  return true;
 }
 
 // Its chunking: whole 64-key tiles, at most kMaxSplitChunks chunks (the merge

@@ -70,8 +70,7 @@ struct PrefillArgs {
 struct VerifyArgs {
   int64_t chunk;
   int nchunks, ncols;
-  int items;  // mi::wide_count: workgroups per KV head
-  int run;    // items of an XCD's run, or 0
+  mi::WideDeal deal;
   int64_t nslots;
   float* part_o;
   float* part_ml;
@@ -626,10 +625,8 @@ mi_status verify_wide_split(const mi_kv* kv, int32_t layer, const _Float16* q, i
   vx.nslots = nchunks;
   vx.part_o = part_o;
   vx.part_ml = part_ml;
-  vx.items = wide_count((int)past, n, (int)chunk);
-  const int wgs = vx.items * kv->G;
-  vx.run = wide_runs(past, n) ? (wgs + 7) / 8 : 0;
-  return launch_verify_wide(a, vx, vx.run ? vx.run * 8 : wgs, stream);
+  vx.deal = wide_deal(kv->G, past, n, chunk, nchunks);
+  return launch_verify_wide(a, vx, vx.deal.grid, stream);
 }
 
 }  // namespace mi

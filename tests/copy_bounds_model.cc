@@ -95,8 +95,8 @@ static long long prefill64_violations(int past, int n, long long cap) {
 
 // The wide verify / split-K prefill (attn_verify_wide_kernel): plan
 // mi::wide_plan (two KV heads); workgroup (row block rb of 16 tokens, chunk
-// c), enumerated by mi::wide_item: keys from kbeg = c * chunk, wave (qb, kp) walking mi::verify_wave64's
-// tiles with the 64-query kernel's copies (K(0) first; then K(min(t + 1,
+// c), placed by mi::wide_place as in the kernel: keys from kbeg = c * chunk,
+// wave (qb, kp) walking mi::verify_wave64's tiles with the 64-query kernel's copies (K(0) first; then K(min(t + 1,
 // nt - 1)) and V(t) at tile 0 and on active tiles, else K(t + 1) when
 // t + 1 < nt and V(t); the max pass copies K only), tile T being rows
 // [kbeg + 64 T, + 64).  Every copy must lie inside `cap` rows, the chunks
@@ -109,16 +109,18 @@ static long long wide_violations(long long past, int n, long long cap) {
   if (wp.chunk % mi::kPrefillBK || wp.nchunks > mi::kMaxSplitChunks ||
       (long long)wp.nchunks * wp.chunk < past + n)
     bad++;
-  // the items name every (row block, chunk) with visible keys exactly once
+  // the workgroups name every (row block, chunk) with visible keys exactly once
+  // per KV head
   const int nrb = (n + 15) / 16;
-  std::vector<char> named((size_t)nrb * wp.nchunks, 0);
-  const int items = mi::wide_count((int)past, n, (int)wp.chunk);
+  std::vector<char> named((size_t)nrb * wp.nchunks * 2, 0);
+  const mi::WideDeal deal = mi::wide_deal(2, past, n, wp.chunk, wp.nchunks);
   // one round of the 256 CUs, where the row blocks alone do not exceed it
-  if (nrb * 2 <= 256 && items * 2 > 256) bad++;
-  for (int i = 0; i < items; i++) {
-      int rb, c;
-      mi::wide_item((int)past, n, (int)wp.chunk, i, rb, c);
-      if (rb < 0 || rb >= nrb || c < 0 || c >= wp.nchunks || named[(size_t)rb * wp.nchunks + c]++) {
+  if (nrb * 2 <= 256 && deal.grid > 256) bad++;
+  for (int i = 0; i < deal.grid; i++) {
+      int rb, c, kvh;
+      if (!mi::wide_place(deal, 2, (int)past, n, (int)wp.chunk, i, rb, c, kvh)) continue;
+      if (rb < 0 || rb >= nrb || c < 0 || c >= wp.nchunks || kvh < 0 || kvh > 1 ||
+          named[((size_t)rb * wp.nchunks + c) * 2 + kvh]++) {
         bad++;
         continue;
       }
@@ -152,9 +154,10 @@ static long long wide_violations(long long past, int n, long long cap) {
   }
   for (int rb = 0; rb < nrb; rb++)
     for (int c = 0; c < wp.nchunks; c++)
-      if (named[(size_t)rb * wp.nchunks + c] !=
-          ((long long)c * wp.chunk < mi::wide_end((int)past, n, rb)))
-        bad++;
+      for (int kvh = 0; kvh < 2; kvh++)
+        if (named[((size_t)rb * wp.nchunks + c) * 2 + kvh] !=
+            ((long long)c * wp.chunk < mi::wide_end((int)past, n, rb)))
+          bad++;
   return bad;
 }
 
@@ -222,7 +225,8 @@ int main() {
   std::printf("split %lld %lld\n", cs, bs);
 
   long long cw = 0, bw = 0;
-  for (long long past : {0LL, 1LL, 63LL, 64LL, 65LL, 700LL, 2048LL, 4096LL, 20000LL, 65536LL,
+  for (long long past : {0LL, 1LL, 63LL, 64LL, 65LL, 700LL, 2048LL, 4096LL, 5000LL, 6500LL,
+                         12287LL, 12288LL, 20000LL, 65536LL,
                          131071LL})
     for (int n = 1; n <= 1100; n += (n < 40 ? 1 : 37)) {
       bw += wide_violations(past, n, round_cap(past + n));
