@@ -156,6 +156,8 @@ mi_status mi_kv_copy_from(mi_kv* dst, const mi_kv* src);
  * h / (H/G); then out *= sigmoid(gate) elementwise when gate != NULL.
  * q, gate, out: [H*D] f16.  Split-K flash-decoding plus a combine kernel, or
  * one launch up to 1024 rows.
+ * out may be q's or gate's buffer (so too in the steps, prefill and verify
+ * below).
  * Semantics: attention_scores/softmax/values_batched + sigmoid_gate_inplace
  * (src/math_util.rs:264-269, 323-383), kernels attn_sdpa_block +
  * attn_sdpa_reduce (src/engine/shaders.metal:1559-1776).  seq_len == 0 gives

@@ -149,7 +149,8 @@ def attn_step_proj(cache, layer: int, q_proj: torch.Tensor, k: torch.Tensor, v: 
 
 def attn_decode(cache, layer: int, q: torch.Tensor, seq_len: int,
                 gate: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
-    """One query token ([H, D] or [H*D]) over rows [0, seq_len) of `layer`."""
+    """One query token ([H, D] or [H*D]) over rows [0, seq_len) of `layer`.
+    out may be q or gate itself, here and in the calls below."""
     out = _check_qgo(cache, q, gate, out, 1)
     _lib.check(_lib.lib().mi_attn_decode(cache._h, cache.slot(layer), _ptr(q), _ptr(gate),
                                          _ptr(out), int(seq_len), _stream()))

@@ -29,6 +29,7 @@
 //    applies the sigmoid gate and writes f16.
 #include <algorithm>
 #include <cstdlib>
+#include <initializer_list>
 #include <type_traits>
 
 #include "common.h"
@@ -1727,8 +1728,22 @@ mi_status wide_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float1
 // Whether n tokens after `past` rows take the one-launch form.
 // MI_ATTN_SPLIT_* and MI_ATTN_DECODE_MERGE (0 or 1) ask for forms of the split
 // launch, MI_ATTN_VERIFY_WIDE=0 for its 4-token groups.
-bool takes_direct(int64_t past, int32_t n, const _Float16* gate, const _Float16* out) {
+// `inputs`: what the launch reads beside the cache and the gate (a gate value is
+// read by the thread that writes its output).  Its workgroups share them
+// (slices of V read the same queries, token pairs the same new rows), so an
+// output in the same memory, which the other forms take - they write it in a
+// later launch, or the prefill grid from the one workgroup that read it - would
+// be stored over what another workgroup has yet to read.
+struct Span {
+  const void* p;
+  size_t bytes;
+};
+bool takes_direct(int64_t past, int32_t n, int H, const _Float16* gate, const _Float16* out,
+                  std::initializer_list<Span> inputs) {
   if (((uintptr_t)gate | (uintptr_t)out) & 7) return false;  // 8-byte accesses here only
+  const uintptr_t o0 = (uintptr_t)out, o1 = o0 + (size_t)n * H * D * sizeof(_Float16);
+  for (const Span& s : inputs)
+    if (s.p && (uintptr_t)s.p < o1 && o0 < (uintptr_t)s.p + s.bytes) return false;
   if (split_knobs().chunk > 0 || split_knobs().gh != 1 || split_knobs().wgs != 256) return false;
   const char* merge = getenv("MI_ATTN_DECODE_MERGE");
   if (n == 1 && merge && *merge) return false;
@@ -1789,7 +1804,10 @@ mi_status run_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16
 mi_status cache_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
                        _Float16* out, int64_t past_pos, int32_t n, hipStream_t stream,
                        const _Float16* k_new = nullptr, const _Float16* v_new = nullptr) {
-  const bool direct = takes_direct(past_pos, n, gate, out);
+  const size_t rows_bytes = (size_t)n * kv->G * D * sizeof(_Float16);
+  const bool direct = takes_direct(
+      past_pos, n, kv->H, gate, out,
+      {{q, (size_t)n * kv->H * D * sizeof(_Float16)}, {k_new, rows_bytes}, {v_new, rows_bytes}});
   if (n > 4 && verify_wide_enabled()) {
     const bool groups = !direct && mi::verify_groups(past_pos, n);
     if (!direct && !groups)
@@ -1895,7 +1913,8 @@ mi_status attend_cache(mi_kv* kv, int32_t layer, const _Float16* q, const _Float
 
 bool attend_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
                    _Float16* out, int64_t past, int32_t n, hipStream_t stream, mi_status* st) {
-  if (!takes_direct(past, n, gate, out)) return false;
+  if (!takes_direct(past, n, kv->H, gate, out, {{q, (size_t)n * kv->H * D * sizeof(_Float16)}}))
+    return false;
   // The workspace an eager split-K call of this size leaves for later captured
   // calls, although this form needs none.
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -2036,7 +2055,14 @@ extern "C" mi_status mi_attn_step_proj(mi_kv* kv, int32_t layer, const float* q_
   const SplitPlan plan = plan_split(rows, 1, kv->G, 1);
   void* ws;
   MI_TRY(mi::kv_workspace(kv, attend_workspace_bytes(kv->G, plan.max_chunks, 1), (hipStream_t)stream, &ws));
-  if (takes_direct(pos, 1, nullptr, (const _Float16*)out)) {
+  const size_t q_bytes = (size_t)kv->H * 2 * D * sizeof(float);
+  const size_t kv_bytes = (size_t)kv->G * D * sizeof(float), w_bytes = D * sizeof(uint16_t);
+  if (takes_direct(pos, 1, kv->H, nullptr, (const _Float16*)out,
+                   {{q_proj, q_bytes},
+                    {k, kv_bytes},
+                    {v, kv_bytes},
+                    {q_norm_w, w_bytes},
+                    {k_norm_w, w_bytes}})) {
     MI_TRY(run_direct(kv, layer, nullptr, nullptr, (_Float16*)out, pos, 1, (hipStream_t)stream,
                       nullptr, nullptr, &x));
     kv->len[layer] = pos + 1;

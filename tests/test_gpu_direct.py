@@ -162,6 +162,62 @@ def test_weights_of_the_split_forms(monkeypatch, past, n):
     assert share <= 0.1
 
 
+@pytest.mark.parametrize("call,past,n", [
+    (step, 0, 1), (step, 300, 1), (step, 5000, 1), (attn_verify, 40, 2), (attn_verify, 300, 4),
+    (attn_verify, 300, 9), (attn_verify, 5000, 9), (attn_verify, 100, 40), (attn_prefill, 0, 17),
+    (attn_prefill, 300, 64), (attn_prefill, 0, 100), (attn_prefill, 50, 333),
+    (attn_prefill, 0, 1100), (attn_prefill, 3000, 100)])
+@pytest.mark.parametrize("buffer", ["q", "gate"])
+def test_output_in_the_buffer_of_an_input(call, past, n, buffer):
+    """The output may take the place of the queries or of the gate, at any
+    length: the calls that would run in one launch, where workgroups share
+    their queries, go to the forms that write the output when all are read."""
+    rng = np.random.default_rng(past + n)
+    rows = past + n
+    k, v = f16(rng, rows, G * D), f16(rng, rows, G * D)
+    q, g = dev(f16(rng, n, H, D)), dev(f16(rng, n, H, D))
+    c = Cache(num_layers=1, capacity=rows)
+    if past:
+        c.upload(0, k[:past], v[:past])
+    announce(f"out in {buffer} {call.__name__} past={past} n={n}")
+    args = (c, 0, q, dev(k[past:]), dev(v[past:]), past)
+    ref = host(call(*args, gate=g)).reshape(n, H, D)
+    out = q if buffer == "q" else g
+    f = attn_step if call is step else call
+    args = (c, 0, q.view(-1) if call is step else q) + args[3:]
+    got = f(*args, gate=g.view(-1) if call is step else g,
+            out=out.view(-1) if call is step else out)
+    assert got.data_ptr() == out.data_ptr()
+    # two forms of the same sums: an f16 ulp of outputs below 4
+    assert_close(host(out).reshape(n, H, D), ref, f"out in {buffer}", atol=2.0 ** -9)
+
+
+@pytest.mark.parametrize("past", [0, 300])
+@pytest.mark.parametrize("buffer", ["k", "v"])
+def test_output_over_the_new_rows(past, buffer):
+    """The same for the new K / V rows, which every workgroup of a head reads
+    when the launch appends them."""
+    rng = np.random.default_rng(past)
+    n = 16
+    rows = past + n
+    k, v = f16(rng, rows, G * D), f16(rng, rows, G * D)
+    q = dev(f16(rng, n, H, D))
+    c = Cache(num_layers=1, capacity=rows)
+    if past:
+        c.upload(0, k[:past], v[:past])
+    announce(f"out over {buffer} past={past}")
+    ref = host(attn_verify(c, 0, q, dev(k[past:]), dev(v[past:]), past))
+    buf = torch.empty(n * H * D, dtype=torch.float16, device="cuda")
+    new = buf[:n * G * D]
+    new.copy_(dev((k if buffer == "k" else v)[past:]).view(-1))
+    pair = (new, dev(v[past:])) if buffer == "k" else (dev(k[past:]), new)
+    got = attn_verify(c, 0, q, *pair, past, out=buf.view(n, H, D))
+    assert_close(got, ref, f"out over {buffer}", atol=2.0 ** -9)
+    kc, vc = c.download(0, rows=n, row0=past)
+    np.testing.assert_array_equal(kc, k[past:])
+    np.testing.assert_array_equal(vc, v[past:])
+
+
 @pytest.mark.parametrize("past,n", [(999, 513), (320, 640), (1030, 1024)])
 def test_split_k_with_row_blocks_of_different_length(monkeypatch, past, n):
     """The split-K prefill where the blocks of 16 tokens see different numbers
