@@ -1751,6 +1751,14 @@ bool takes_direct(int64_t past, int32_t n, int H, const _Float16* gate, const _F
   return mi::direct_rows(past, n);
 }
 
+// Slices of V while the launch has fewer workgroups than CUs.  Measured (us, 4 /
+// 2 / 1 slices): no past, 64 tokens 3.6 / 4.3 / 5.7, 128 tokens 5.9 / 5.1 / 6.5,
+// 333 tokens 15.6 / 12.5 / 11.3.
+int direct_slices(int G, int32_t n) {
+  const int wgs = (n + 1) / 2 * G;
+  return wgs * 4 <= 256 ? 4 : wgs * 2 <= 256 ? 2 : 1;
+}
+
 // Most new rows the one-launch form appends itself (every workgroup of a head
 // writes them); more go in a launch before it.
 constexpr int kDirectAppend = 16;
@@ -1758,7 +1766,7 @@ constexpr int kDirectAppend = 16;
 mi_status run_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
                      _Float16* out, int64_t past, int32_t n, hipStream_t stream,
                      const _Float16* k_new, const _Float16* v_new, const ProjArgs* proj,
-                     bool grid_precision = false) {
+                     bool prefill = false) {
   if (k_new && n > kDirectAppend) {
     MI_TRY(mi::kv_append_rows(kv, layer, k_new, v_new, past, n, stream));
     k_new = v_new = nullptr;
@@ -1786,13 +1794,11 @@ mi_status run_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16
       default: return launch_direct_proj<4>(a, stream, *proj);
     }
   }
-  // Slices of V while the launch has fewer workgroups than CUs.  Measured
-  // (us, NDB = 4 / 8 / 16): no past, 64 tokens 3.6 / 4.3 / 5.7, 128 tokens 5.9 /
-  // 5.1 / 6.5, 333 tokens 15.6 / 12.5 / 11.3.
-  const int wgs = (n + 1) / 2 * kv->G;
-  if (wgs * 4 <= 256) return launch_direct<4>(a, stream);
-  if (wgs * 2 <= 256) return launch_direct<8>(a, stream);
-  return grid_precision ? launch_direct<16, false>(a, stream) : launch_direct<16>(a, stream);
+  switch (direct_slices(kv->G, n)) {
+    case 4: return launch_direct<4>(a, stream);
+    case 2: return launch_direct<8>(a, stream);
+  }
+  return prefill ? launch_direct<16, false>(a, stream) : launch_direct<16>(a, stream);
 }
 
 // Verify / decode over the cache: n query tokens at positions past_pos ..
@@ -1915,16 +1921,20 @@ bool attend_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* 
                    _Float16* out, int64_t past, int32_t n, hipStream_t stream, mi_status* st) {
   if (!takes_direct(past, n, kv->H, gate, out, {{q, (size_t)n * kv->H * D * sizeof(_Float16)}}))
     return false;
+  // Long pasts next to n: the split-K form serves them as well.  In one slice of
+  // V, where the precision of its weights would have to be paid for (TILE), it is
+  // the faster one: 160 tokens after 2500 rows 29.6 us against 30.8.
+  const bool split = past >= 2048 && past >= 2 * (int64_t)n;
+  if (split && direct_slices(kv->G, n) == 1) return false;
   // The workspace an eager split-K call of this size leaves for later captured
   // calls, although this form needs none.
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   void* ws;
-  const bool split = past >= 2048 && past >= 2 * (int64_t)n;  // else what the grid would run
   if (split && hipStreamIsCapturing(stream, &cs) == hipSuccess &&
       cs == hipStreamCaptureStatusNone &&
       (*st = mi::kv_workspace(kv, wide_launch(kv->G, past, n).ws_bytes, stream, &ws)) != MI_OK)
     return true;
-  *st = run_direct(kv, layer, q, gate, out, past, n, stream, nullptr, nullptr, nullptr, !split);
+  *st = run_direct(kv, layer, q, gate, out, past, n, stream, nullptr, nullptr, nullptr, true);
   return true;
 }
 
