@@ -1468,7 +1468,8 @@ mi_status run_split(const _Float16* k, const _Float16* v, const int32_t* offsets
                     void* ws, size_t ws_bytes, hipStream_t stream,
                     const AppendRows& app = AppendRows(), const ProjArgs* proj = nullptr,
                     const mi_kv* kv = nullptr, int ntok = 0) {
-  const SplitPlan plan = plan_split(max_len, batch, G, nq);
+  const SplitPlan plan = ntok ? mi::plan_groups(max_len, (int)batch, G, split_knobs())
+                              : plan_split(max_len, batch, G, nq);
   SplitArgs a;
   a.mcnt = nullptr;
   a.k = k;
@@ -1828,7 +1829,9 @@ mi_status cache_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float
     size_t need = wide_launch(kv->G, past_pos, n).ws_bytes;
     if (groups)
       need = std::max(need, split_workspace_bytes(
-                                ng, kv->G, plan_split(past_pos + n, ng, kv->G, 4).max_chunks, 4));
+                                ng, kv->G,
+                                mi::plan_groups(past_pos + n, ng, kv->G, split_knobs()).max_chunks,
+                                4));
     void* ws;
     MI_TRY(mi::kv_workspace(kv, need, stream, &ws));
     if (groups) {

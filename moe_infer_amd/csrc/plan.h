@@ -366,4 +366,26 @@ inline SplitPlan plan_split(int64_t max_len, int64_t batch, int G, int nq, const
   return p;
 }
 
+// Chunking of a verify by `ng` groups of four tokens (the split launch's z
+// planes): chunks whose workgroups all run at once, not one more (9 tokens after
+// 16300 rows in 43 chunks of two heads, 258 workgroups, took 38.2 us, in 32
+// chunks 25.8), and a chunk count, padded with empty chunks where those still
+// fit, that puts the groups of a chunk on one XCD (blockIdx % 8), whose L2 then
+// reads its K/V once: 13 tokens after 19314 rows in 31 chunks 37.0 us, padded to
+// 32 29.0; after 17000 rows in 27 chunks 33.9, padded to 28 28.4.
+inline SplitPlan plan_groups(int64_t rows, int ng, int G, const SplitKnobs& k) {
+  SplitPlan p = plan_split(rows, ng, G, 4, k);
+  const int step = 32 * p.nwh, wgs = 256;
+  if (k.chunk <= 0)
+    while (p.max_chunks * ng * G > wgs && p.chunk < rows) {
+      p.chunk += step;
+      p.max_chunks = (int)((rows + p.chunk - 1) / p.chunk);
+    }
+  int lanes = 8;  // chunks to a round of the XCDs
+  while (lanes > 1 && lanes / 2 * G % 8 == 0) lanes /= 2;
+  const int padded = (p.max_chunks + lanes - 1) / lanes * lanes;
+  if (padded * ng * G <= wgs) p.max_chunks = padded;
+  return p;
+}
+
 }  // namespace mi

@@ -224,6 +224,20 @@ int main() {
     }
   std::printf("split %lld %lld\n", cs, bs);
 
+  // verify by token groups: the chunks cover the rows, a grid of one round of
+  // workgroups where one chunk each would be
+  long long cg = 0, bg = 0;
+  for (int G : {1, 2, 3, 4, 8})
+    for (int ng = 2; ng <= 4; ng++)
+      for (long long rows = 1; rows <= 20480; rows += (rows < 600 ? 1 : 13)) {
+        const mi::SplitPlan p = mi::plan_groups(rows, ng, G, mi::SplitKnobs{1, 256, 0});
+        if (p.chunk % (32 * p.nwh) || p.max_chunks > mi::kMaxSplitChunks ||
+            (long long)p.chunk * p.max_chunks < rows || p.max_chunks * ng * G > 256)
+          bg++;
+        cg++;
+      }
+  std::printf("groups %lld %lld\n", cg, bg);
+
   long long cw = 0, bw = 0;
   for (long long past : {0LL, 1LL, 63LL, 64LL, 65LL, 700LL, 2048LL, 4096LL, 5000LL, 6500LL,
                          12287LL, 12288LL, 20000LL, 65536LL,

@@ -65,3 +65,10 @@ def test_wide_verify_tiles_stay_inside_the_allocation(model_output):
     chunks whole tiles covering every row, each token's visible keys walked."""
     cases, bad = model_output["wide"]
     assert cases > 500 and bad == 0
+
+
+def test_token_groups_run_in_one_round(model_output):
+    """A verify by token groups: chunks that cover every row, in no more
+    workgroups than the 256 CUs take at once."""
+    cases, bad = model_output["groups"]
+    assert cases > 20000 and bad == 0
