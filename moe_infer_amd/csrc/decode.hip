@@ -44,14 +44,15 @@ constexpr float kNegBig = -1e30f;
 // computes itself (no plan launch); larger batches run ragged_plan_kernel.
 constexpr int kFusedPlan = 256;
 
-// Ragged batches of up to kChunkTiles tiles per spare workgroup (grid minus
-// sequences) are dealt out by chunks of one sequence, ceil(tiles / spare) tiles
-// each, so that no workgroup crosses into a second sequence: a crossing runs
-// the whole chain (Q, K, V, merge, store) twice, and with a tile or two per
-// wave that chain is the launch.  Per call
-// (us, against tiles dealt evenly across sequences): 8 sequences of 100..3000
-// rows 25.7 -> 15.5, 2 of 3000 32.5 -> 15.7, 32 of 500..2000 26.4 -> 24.5, 100 of
-// 50..200 24.7 -> 18.1.
+// Ragged batches of more tiles than workgroups, up to kChunkTiles per spare
+// workgroup (grid minus sequences), are dealt out by chunks of one sequence,
+// ceil(tiles / spare) tiles each, so that no workgroup crosses into a second
+// sequence: a crossing runs the whole chain (Q, K, V, merge, store) twice, and
+// with a tile or two per wave that chain is the launch.  Per call (us, against
+// tiles dealt evenly across sequences): 8 sequences of 100..3000 rows 25.7 ->
+// 15.5, 2 of 3000 32.5 -> 15.7, 32 of 500..2000 26.4 -> 24.5, 100 of 50..200 24.7
+// -> 18.1.  Up to one tile per workgroup nothing crosses, and the second scan
+// that the chunks need would cost 0.6 us (16 of 1..60 rows 12.0 -> 12.9).
 constexpr int kChunkTiles = 16;
 
 struct SplitArgs {
@@ -461,7 +462,7 @@ attn_split_kernel(SplitArgs a, X x) {
         };
         int32_t carry = scan();
         const int32_t spare = (int32_t)gridDim.x - a.batch;
-        if (spare > 0 && carry <= kChunkTiles * spare) {
+        if (carry > (int32_t)gridDim.x && spare > 0 && carry <= kChunkTiles * spare) {
           per = max(1, (carry + spare - 1) / spare);
 #pragma unroll
           for (int c = 0; c < kFusedPlan / 64; c++) n[c] = (n[c] + per - 1) / per;
@@ -1250,6 +1251,7 @@ attn_combine_kernel(CombineArgs a) {
 // Workgroup x < nw = min(nwg, T) of the split took tiles [x T / nw,
 // (x+1) T / nw), so tile t is in workgroup ceil((t+1) nw / T) - 1 and the
 // partials of sequence s are in slots first + s .. last + s.
+template <int MAXB>
 __global__ void __launch_bounds__(D)
 attn_combine_flat_kernel(CombineArgs a) {
   const int c = blockIdx.x, kvh = blockIdx.y, s = blockIdx.z, d = threadIdx.x;
@@ -1271,10 +1273,11 @@ attn_combine_flat_kernel(CombineArgs a) {
   const float* ml = a.part_ml + slot0 * 2;
   const float* po = a.part_o + slot0 * D + d;
   float M = kNegBig, L = 0.f, o = 0.f;
-  // kB partials are loaded per batch, all before their use: 8, or 16 where a
-  // sequence has more (a small batch: 8 sequences of 1550 rows 25.7 -> 16.0 us
-  // per call with the chunks of one sequence; 16 for all cost 200 sequences of
-  // two partials 45 -> 50 us).
+  // kB partials are loaded per batch, all before their use: 8, or 16 (MAXB)
+  // where a sequence has more (a small batch: 8 sequences of 1550 rows 25.7 ->
+  // 16.0 us per call with the chunks of one sequence; 16 for all cost 200
+  // sequences of two partials 45 -> 50 us, and a kernel that holds both 256
+  // sequences of 250..500 rows 53 -> 56).
   auto merge = [&](auto batch) {
     constexpr int kB = decltype(batch)::value;
     for (int64_t c0 = 0; c0 < nch; c0 += kB) {
@@ -1301,8 +1304,8 @@ attn_combine_flat_kernel(CombineArgs a) {
       }
     }
   };
-  if (nch <= 8) merge(std::integral_constant<int, 8>{});
-  else merge(std::integral_constant<int, 16>{});
+  if (MAXB == 8 || nch <= 8) merge(std::integral_constant<int, 8>{});
+  else merge(std::integral_constant<int, MAXB>{});
   float r = (L > 0.f) ? o / L : 0.f;
   if (bad) r = __builtin_nanf("");
   const int hq = kvh * 8 + c;
@@ -1580,8 +1583,10 @@ mi_status run_split(const _Float16* k, const _Float16* v, const int32_t* offsets
   c.batch = (int)batch;
   c.ntok = ntok;
   if (lengths) {
-    MI_HIP(mi::launch("attn_combine", attn_combine_flat_kernel, dim3(8, G, (unsigned)batch),
-                      dim3(D), 0, stream, c));
+    // (128 workgroups per head leave up to 32 sequences four partials or more each)
+    MI_HIP(mi::launch("attn_combine",
+                      batch <= 32 ? attn_combine_flat_kernel<16> : attn_combine_flat_kernel<8>,
+                      dim3(8, G, (unsigned)batch), dim3(D), 0, stream, c));
     return MI_OK;
   }
   if (ntok) {

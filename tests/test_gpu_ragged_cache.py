@@ -47,15 +47,28 @@ def test_ragged_matches_oracle(lengths):
     assert np.all(o[lengths == 0] == 0)
 
 
-@pytest.mark.parametrize("lengths", [
-    [16 * 127 * 32], [16 * 127 * 32 + 1],  # the last length dealt by chunks, the first by tiles
-    [0, 40, 0, 0, 700, 1, 0],              # chunks skip empty sequences
-    [0, 0, 0],                             # nothing to attend
-    [33] * 127, [33] * 128,                # one spare workgroup, none
-    [16 * 32 + 5] * 120 + [0, 9]])         # chunks of 16 tiles and the rest of a sequence
-def test_ragged_chunks_of_one_sequence(lengths):
-    """Batches of few tiles go by chunks of a sequence (2 KV heads: 128
-    workgroups a head), each against the oracle."""
+def dealt_by_chunks(lengths, grid=128):
+    """The split kernel's rule for a batch of up to 256 sequences (2 KV heads: 128
+    workgroups a head): chunks of one sequence, or tiles across sequences."""
+    tiles, spare = sum((n + 31) // 32 for n in lengths), grid - len(lengths)
+    return tiles > grid and spare > 0 and tiles <= 16 * spare
+
+
+@pytest.mark.parametrize("lengths,chunks", [
+    ([128 * 32], False), ([128 * 32 + 1], True),             # more tiles than workgroups
+    ([16 * 127 * 32], True), ([16 * 127 * 32 + 1], False),   # 16 tiles per spare workgroup
+    ([0, 40, 0, 0, 700, 1, 0], False),                       # one tile per workgroup
+    ([0, 3000, 0, 0, 2500, 1, 0], True),                     # chunks skip empty sequences
+    ([0, 0, 0], False),                                      # nothing to attend
+    ([0] * 40 + [1] * 24 + [5000], True),                    # two 64-lane steps of the scans
+    ([50 + 14 * (i % 11) for i in range(100)], True),
+    ([40] * 99 + [8000], True), ([40] * 99 + [8001], False),  # chunks of 16 tiles, the last length
+    ([1] * 118 + [20 * 32], True),                           # 16 tiles and the rest, a nearly full grid
+    ([33] * 119, False), ([33] * 127, False), ([33] * 128, False)])  # few spare workgroups, none
+def test_ragged_chunks_of_one_sequence(lengths, chunks):
+    """Batches of few tiles go by chunks of a sequence, others by tiles, each
+    against the oracle."""
+    assert dealt_by_chunks(lengths) == chunks
     announce(f"ragged chunks batch={len(lengths)} rows={sum(lengths)}")
     rng = np.random.default_rng(sum(lengths) + len(lengths))
     lengths = np.array(lengths, np.int32)
