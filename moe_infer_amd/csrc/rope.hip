@@ -164,6 +164,11 @@ __device__ __forceinline__ void k_rows(const RopeArgs& a, int item, float* lds) 
     sincosf((float)(a.pos + row0 + i) * a.inv_freq[p], &sn, &cs);
     tab[idx] = float2{cs, sn};
   }
+  // the wave's lanes read each other's entries below: LDS serves a wave in
+  // order, this keeps the compiler to it
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   const bool rot = 4 * lane < 2 * rh;
   const int p0 = 4 * lane < rh ? 4 * lane : 4 * lane - rh;
 #pragma unroll
