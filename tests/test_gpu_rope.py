@@ -217,22 +217,27 @@ def test_step_proj_matches_oracle_chain(pos):
         np.testing.assert_array_equal(v0, prev_v)
 
 
-@pytest.mark.parametrize("rot", [0, 128, 256])
-def test_step_proj_rotary_dims(rot):
+# one launch up to 1024 rows (8 columns a lane), the split kernel above (4)
+@pytest.mark.parametrize("pos", [300, 1500])
+@pytest.mark.parametrize("rot", [0, 64, 128, 192, 256])
+def test_step_proj_rotary_dims(rot, pos):
     from moe_infer_amd import attn_step_proj
-    announce(f"attn_step_proj rot={rot}")
-    rng = np.random.default_rng(rot)
-    pos = 300
+    announce(f"attn_step_proj rot={rot} pos={pos}")
+    rng = np.random.default_rng(rot + pos)
     q_proj, k, v, qw, kw = inputs(rng, 1)
     prev_k = rng.standard_normal((pos, G * D)).astype(np.float16)
     prev_v = rng.standard_normal((pos, G * D)).astype(np.float16)
-    c = Cache(num_layers=1, capacity=512)
+    c = Cache(num_layers=1, capacity=pos + 1)
     c.upload(0, prev_k, prev_v)
     out = attn_step_proj(c, 0, torch.from_numpy(q_proj[0]).cuda(), torch.from_numpy(k[0]).cuda(),
                          torch.from_numpy(v[0]).cuda(), qw.cuda(), kw.cuda(), pos,
                          rotary_dim=rot)
-    ref, _ = step_proj_reference(q_proj[0], k[0], v[0], qw, kw, prev_k, prev_v, pos, rot)
-    assert_close(out, ref, f"step_proj rot={rot}")
+    ref, kref = step_proj_reference(q_proj[0], k[0], v[0], qw, kw, prev_k, prev_v, pos, rot)
+    assert_close(out, ref, f"step_proj rot={rot} pos={pos}")
+    kc, vc = c.download(0, rows=1, row0=pos)
+    assert_within_one_ulp(kc, kref.reshape(1, G * D), f"step_proj k row rot={rot} pos={pos}",
+                          f32_slack=True)
+    np.testing.assert_array_equal(vc.view(np.uint16), f16_bits(v[0]).reshape(1, G * D))
 
 
 def test_step_proj_sequence_equals_two_kernel_route():
