@@ -1661,14 +1661,13 @@ __global__ void __launch_bounds__(256) attn_combine_rows_kernel(CombineArgs a) {
   *(f16x4*)(a.out + oidx) = h;
 }
 
-// Wide verify for more than 4 query tokens (MI_ATTN_VERIFY_WIDE=0, read at
-// each call, turns it off): one split pass that reads every K/V tile once
-// per 16 tokens (attn_prefill64_kernel's MFMA tiles over key chunks), then
-// the combine, instead of one split-K launch pair per 4-token group.
-bool verify_wide_enabled() {
-  const char* e = getenv("MI_ATTN_VERIFY_WIDE");
+// A form's switch, read at each call: off when set to 0.
+bool switched_on(const char* name) {
+  const char* e = getenv(name);
   return !(e && *e && atoi(e) == 0);
 }
+// More than 4 query tokens in forms other than a launch pair per four tokens.
+bool verify_wide_enabled() { return switched_on("MI_ATTN_VERIFY_WIDE"); }
 
 // The wide verify's plan (mi::wide_plan) and the workspace its partials
 // (O, m, l) take.
@@ -1731,9 +1730,9 @@ mi_status wide_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float1
   return MI_OK;
 }
 
-// Whether n tokens after `past` rows take the one-launch form.
-// MI_ATTN_SPLIT_* and MI_ATTN_DECODE_MERGE (0 or 1) ask for forms of the split
-// launch, MI_ATTN_VERIFY_WIDE=0 for its 4-token groups.
+// Whether n tokens after `past` rows take the one-launch form.  MI_ATTN_DIRECT=0
+// (read at each call) turns it off; MI_ATTN_SPLIT_* and, for one token,
+// MI_ATTN_DECODE_MERGE (0 or 1) ask for forms of the split launch.
 // `inputs`: what the launch reads beside the cache and the gate (a gate value is
 // read by the thread that writes its output).  Its workgroups share them
 // (slices of V read the same queries, token pairs the same new rows), so an
@@ -1746,6 +1745,7 @@ struct Span {
 };
 bool takes_direct(int64_t past, int32_t n, int H, const _Float16* gate, const _Float16* out,
                   std::initializer_list<Span> inputs) {
+  if (!mi::direct_rows(past, n)) return false;
   if (((uintptr_t)gate | (uintptr_t)out) & 7) return false;  // 8-byte accesses here only
   const uintptr_t o0 = (uintptr_t)out, o1 = o0 + (size_t)n * H * D * sizeof(_Float16);
   for (const Span& s : inputs)
@@ -1753,8 +1753,7 @@ bool takes_direct(int64_t past, int32_t n, int H, const _Float16* gate, const _F
   if (split_knobs().chunk > 0 || split_knobs().gh != 1 || split_knobs().wgs != 256) return false;
   const char* merge = getenv("MI_ATTN_DECODE_MERGE");
   if (n == 1 && merge && *merge) return false;
-  if (n > 4 && !verify_wide_enabled()) return false;
-  return mi::direct_rows(past, n);
+  return switched_on("MI_ATTN_DIRECT");
 }
 
 // Slices of V while the launch has fewer workgroups than CUs.  Measured (us, 4 /
@@ -1809,23 +1808,26 @@ mi_status run_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16
 
 // Verify / decode over the cache: n query tokens at positions past_pos ..
 // past_pos+n-1, rows [0, past_pos+n) already in the cache.
-// With k_new / v_new, the n new rows [past_pos, past_pos + n) are appended
-// by the split kernels themselves (each token group appends its own rows,
-// which precede every read of them; the wide form appends them all in a
-// launch of their own first); the caller has grown the cache.
+// With k_new / v_new, the n new rows [past_pos, past_pos + n) are appended by
+// the attention kernels themselves, each workgroup the rows that it reads before
+// it does (in one launch for all groups, all new rows of its chunk); the wide
+// form, and the one-launch form of more than kDirectAppend tokens, append them
+// in a launch of their own first.  The caller has grown the cache.
 mi_status cache_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
                        _Float16* out, int64_t past_pos, int32_t n, hipStream_t stream,
                        const _Float16* k_new = nullptr, const _Float16* v_new = nullptr) {
   const size_t rows_bytes = (size_t)n * kv->G * D * sizeof(_Float16);
+  const bool wide = n > 4 && verify_wide_enabled();
   // (in one slice of V the wide pass is the faster one from about 2400 rows: 129
-  // tokens after 2900 rows 39.7 us against 37.8, after 2100 33.0 against 36.5)
+  // tokens after 2900 rows 33.9 us against 39.7, after 2100 36.5 against 33.0)
   const bool direct =
-      (past_pos < 2400 || direct_slices(kv->G, n) > 1) &&
+      (n <= 4 || wide) && (past_pos < 2400 || direct_slices(kv->G, n) > 1) &&
       takes_direct(past_pos, n, kv->H, gate, out,
                    {{q, (size_t)n * kv->H * D * sizeof(_Float16)}, {k_new, rows_bytes},
                     {v_new, rows_bytes}});
-  if (n > 4 && verify_wide_enabled()) {
-    const bool groups = !direct && mi::verify_groups(past_pos, n);
+  if (wide) {
+    const bool groups =
+        !direct && mi::verify_groups(past_pos, n) && switched_on("MI_ATTN_VERIFY_GROUPS");
     if (!direct && !groups)
       return wide_attend(kv, layer, q, gate, out, past_pos, n, stream, k_new, v_new);
     // (the wide form's workspace too: a later captured call may count on what

@@ -124,14 +124,26 @@ def test_verify_matches_causal_oracle(n, past):
     assert c.len(0) == past + n
 
 
-@pytest.mark.parametrize("n,past", [(16, 20000), (8, 20000)])
+@pytest.mark.parametrize("n,past", [(5, 0), (6, 63), (8, 300), (9, 1000), (16, 61),
+                                    (13, 4093), (12, 4096), (16, 20000)])
+def test_wide_verify_of_one_row_block(n, past, monkeypatch):
+    """The wide pass with up to 16 tokens, at lengths that the one-launch form
+    and the token groups take by default."""
+    monkeypatch.setenv("MI_ATTN_DIRECT", "0")
+    monkeypatch.setenv("MI_ATTN_VERIFY_GROUPS", "0")
+    test_verify_matches_causal_oracle(n, past)
+
+
+@pytest.mark.parametrize("n,past", [(16, 20000), (8, 20000), (12, 24000)])
 def test_wide_verify_rising_scores_and_grouped_form(n, past, monkeypatch):
-    """5..16 tokens run the wide verify (the prefill's MFMA tiles over key
-    chunks of a few 64-key tiles).  Keys whose scores rise steeply along the
+    """5..16 tokens in the wide verify (the prefill's MFMA tiles over key
+    chunks of a few 64-key tiles; the token groups that serve the shorter
+    contexts off).  Keys whose scores rise steeply along the
     context put a chunk's later tiles far above its first tile's max (the
     fixed reference max), so the workgroups take the restart path; the
-    result matches the oracle and the grouped 4-token form
-    (MI_ATTN_VERIFY_WIDE=0)."""
+    result matches the oracle, and so do the token groups in one launch and
+    the launch pairs of four tokens (MI_ATTN_VERIFY_WIDE=0)."""
+    monkeypatch.setenv("MI_ATTN_VERIFY_GROUPS", "0")
     announce(f"wide verify rising n={n} past={past}")
     rng = np.random.default_rng(n + past)
     L = past + n
@@ -153,6 +165,10 @@ def test_wide_verify_rising_scores_and_grouped_form(n, past, monkeypatch):
     out = attn_verify(c, 0, dev(q), dev(kall[past:]), dev(vall[past:]), past, gate=dev(g))
     ref = O.causal(q, kall, vall, past, gate=g)
     assert_close(out, ref, f"wide verify rising n={n}")
+    monkeypatch.delenv("MI_ATTN_VERIFY_GROUPS")
+    c.set_pos(past)
+    out = attn_verify(c, 0, dev(q), dev(kall[past:]), dev(vall[past:]), past, gate=dev(g))
+    assert_close(out, ref, f"verify by groups rising n={n}")
     monkeypatch.setenv("MI_ATTN_VERIFY_WIDE", "0")
     c.set_pos(past)
     grouped = attn_verify(c, 0, dev(q), dev(kall[past:]), dev(vall[past:]), past, gate=dev(g))
@@ -267,14 +283,17 @@ def test_graph_replay_of_steps_matches_eager():
                  "graph step vs oracle")
 
 
-def test_graph_replay_of_wide_verify_and_split_prefill():
-    """The wide verify (8 tokens) and the split-K prefill (40 tokens after a
-    past of 6008 rows), each an append, a split pass and a merge, captured in
-    one HIP graph after an eager call sized the workspace: every replay, with
-    eager work between, equals the eager outputs bit for bit, and those match
-    the oracle."""
+@pytest.mark.parametrize("form", ["wide", "groups"])
+def test_graph_replay_of_wide_verify_and_split_prefill(form, monkeypatch):
+    """The verify of 8 tokens (in the wide pass, and by token groups, the
+    default at this length) and the split-K prefill (40 tokens after a
+    past of 6008 rows), captured in one HIP graph after an eager call sized
+    the workspace: every replay, with eager work between, equals the eager
+    outputs bit for bit, and those match the oracle."""
     from moe_infer_amd import attn_prefill
-    announce("graph replay of wide verify / split-K prefill")
+    if form == "wide":
+        monkeypatch.setenv("MI_ATTN_VERIFY_GROUPS", "0")
+    announce(f"graph replay of verify ({form}) / split-K prefill")
     rng = np.random.default_rng(33)
     L, n8, n40 = 6000, 8, 40
     k, v = f16(rng, L + n8 + n40, G * D), f16(rng, L + n8 + n40, G * D)
@@ -355,11 +374,48 @@ def test_graph_survives_workspace_growth_on_the_same_handle():
         assert torch.equal(ref.view(torch.int16), out.view(torch.int16)), f"replay {r}"
 
 
-def test_gate_extremes_decode_and_prefill():
+@pytest.mark.parametrize("direct,groups,split", [("1", "1", "1"), ("0", "1", "1"), ("0", "0", "0")])
+@pytest.mark.parametrize("n", [1, 4, 8, 40, 200])
+def test_weights_below_the_normal_range_of_f16(n, direct, groups, split, monkeypatch):
+    """One key 15.3 (base 2) above a thousand others: their weights, 2^-15.3, are
+    f16 subnormals (step 2^-24).  Row sum and PV product must hold the same
+    weights: columns where every value is 1 give 1 (one f16 ulp, 2^-11); where
+    the large key's value is 0 the others' sum remains, within the rounding of
+    a weight (2^-25 of 2^-15.3, 0.12 %) and of the output (0.05 %).  A flush to
+    zero in the sum alone would give 1.025, in the product 0."""
+    from moe_infer_amd import attn_prefill
+    for name, value in (("DIRECT", direct), ("VERIFY_GROUPS", groups), ("PREFILL_SPLIT", split)):
+        monkeypatch.setenv(f"MI_ATTN_{name}", value)
+    announce(f"subnormal weights n={n} direct={direct} groups={groups} split={split}")
+    past = 1000
+    rows = past + n
+    k = np.zeros((rows, G, D), np.float16)
+    k[0, :, 0] = 10.6
+    v = np.ones((rows, G, D), np.float16)
+    v[0, :, 1::2] = 0
+    k, v = k.reshape(rows, -1), v.reshape(rows, -1)
+    q = np.zeros((n, H, D), np.float16)
+    q[:, :, 0] = 16
+    c = filled_cache(k[:past], v[:past], capacity=rows)
+    if n == 1:
+        out = attn_step(c, 0, dev(q), dev(k[past:]), dev(v[past:]), past)
+    else:
+        call = attn_verify if n <= 16 else attn_prefill
+        out = call(c, 0, dev(q), dev(k[past:]), dev(v[past:]), past)
+    out = host(out).reshape(n, H, D).astype(np.float64)
+    p = np.exp(-float(np.float16(10.6))) * (past + np.arange(n))[:, None, None]
+    assert np.abs(out[:, :, 0::2] - 1).max() <= 2.0 ** -11
+    assert np.abs(out[:, :, 1::2] / (p / (1 + p)) - 1).max() <= 2e-3
+
+
+@pytest.mark.parametrize("direct", ["1", "0"])
+def test_gate_extremes_decode_and_prefill(direct, monkeypatch):
     """Gate logits far in both tails (sigmoid -> 0 and -> 1, including values
-    whose exponential overflows f32) and around 0, for the decode combine and
-    the prefill epilogue, against the oracle's x / (1 + e^-g)."""
-    announce("gate extremes")
+    whose exponential overflows f32) and around 0, for the one-launch form, and
+    without it the decode combine and the prefill epilogue, against the
+    oracle's x / (1 + e^-g)."""
+    monkeypatch.setenv("MI_ATTN_DIRECT", direct)
+    announce(f"gate extremes direct={direct}")
     from moe_infer_amd import attn_prefill
     rng = np.random.default_rng(21)
     L = 300
@@ -380,13 +436,18 @@ def test_gate_extremes_decode_and_prefill():
 
 
 @pytest.mark.parametrize("Hq,Gk", [(32, 4), (8, 1)])
-def test_other_head_counts(Hq, Gk):
+@pytest.mark.parametrize("form", ["default", "general"])
+def test_other_head_counts(Hq, Gk, form, monkeypatch):
     """Head counts other than 16 / 2 (eight query heads per KV head, the
-    kernels' group size): decode, verify of 4 and 12 tokens (the grouped and
-    wide forms) and prefill (its grid, and its split-K form after a long
-    past) against the oracle."""
+    kernels' group size): decode, verify of 4 and 12 tokens (token groups) and
+    prefill (one launch) against the oracle; then, with the one-launch form
+    and the token groups off, the same through the wide pass, the prefill grid
+    and, after a long past, its split-K form."""
     from moe_infer_amd import attn_prefill
-    announce(f"head counts H={Hq} G={Gk}")
+    if form == "general":
+        monkeypatch.setenv("MI_ATTN_DIRECT", "0")
+        monkeypatch.setenv("MI_ATTN_VERIFY_GROUPS", "0")
+    announce(f"head counts H={Hq} G={Gk} {form}")
     rng = np.random.default_rng(Hq + Gk)
     L = 3000
     k, v = f16(rng, L + 64, Gk * D), f16(rng, L + 64, Gk * D)
@@ -402,7 +463,7 @@ def test_other_head_counts(Hq, Gk):
         out = attn_verify(c, 0, dev(q), dev(k[L:L + n]), dev(v[L:L + n]), L, gate=dev(g))
         ref = O.causal(q, k[:L + n], v[:L + n], L, gate=g, H=Hq, G=Gk)
         assert_close(out, ref, f"verify n={n} H={Hq}")
-    for past, n in ((0, 300), (2500, 40)):  # the grid; the split-K form
+    for past, n in ((0, 300), (2500, 40)):  # general: the grid; the split-K form
         q = f16(rng, n, Hq, D)
         c.set_pos(past)
         out = attn_prefill(c, 0, dev(q), dev(k[past:past + n]), dev(v[past:past + n]), past)

@@ -218,10 +218,12 @@ def test_output_over_the_new_rows(past, buffer):
     np.testing.assert_array_equal(vc, v[past:])
 
 
-@pytest.mark.parametrize("past,n", [(999, 513), (320, 640), (1030, 1024)])
+@pytest.mark.parametrize("past,n", [(999, 513), (480, 640), (1030, 1024),
+                                    (777, 777), (9000, 49), (12500, 40), (30000, 17)])
 def test_split_k_with_row_blocks_of_different_length(monkeypatch, past, n):
     """The split-K prefill where the blocks of 16 tokens see different numbers
-    of chunks: against the prefill grid (the bound of that comparison in
+    of chunks (last chunks of more blocks than fit one at 480 + 640 and 777 +
+    777 rows), in each order of its workgroups: against the prefill grid (the bound of that comparison in
     test_gpu_prefill) and, at rows on both sides of a block, the oracle."""
     rng = np.random.default_rng(past + n)
     rows = past + n

@@ -14,10 +14,26 @@ pytestmark = pytest.mark.gpu
 H, G, D = 16, 2, 256
 
 
+@pytest.fixture
+def grid(monkeypatch):
+    """Calls run the prefill grid at every size, not the one-launch form of
+    short prompts nor the split over the past."""
+    monkeypatch.setenv("MI_ATTN_DIRECT", "0")
+    monkeypatch.setenv("MI_ATTN_PREFILL_SPLIT", "0")
+
+
+@pytest.fixture(params=["grid", "default"])
+def form(request):
+    """The prefill grid, and what a call of that size runs by default."""
+    if request.param == "grid":
+        request.getfixturevalue("grid")
+    return request.param
+
+
 @pytest.mark.parametrize("n,past", [(1, 0), (2, 0), (5, 3), (64, 0), (127, 0), (128, 0),
                                     (129, 0), (300, 0), (200, 77), (256, 64), (130, 1000)])
 @pytest.mark.parametrize("gated", [True, False])
-def test_prefill_matches_oracle(n, past, gated):
+def test_prefill_matches_oracle(n, past, gated, form):
     announce(f"prefill n={n} past={past} gated={gated}")
     rng = np.random.default_rng(7 * n + past)
     kp, vp = f16(rng, past, G * D), f16(rng, past, G * D)
@@ -57,7 +73,7 @@ def test_prefill_4k_sampled_rows_and_decode_consistency():
     assert np.all(np.isfinite(out))
 
 
-def test_prefill_rising_scores():
+def test_prefill_rising_scores(form):
     """Scores that rise by ~20 (base 2) per 64-key tile: the steady-state
     tiles exceed the running reference max far enough that the kernel must
     redo them with the new row max (its weights would leave f16 range), and
@@ -82,7 +98,7 @@ def test_prefill_rising_scores():
 
 
 @pytest.mark.parametrize("past,n", [(308, 141), (200, 56), (31, 162)])
-def test_prefill_cache_full_to_capacity(past, n):
+def test_prefill_cache_full_to_capacity(past, n, form):
     """The cache holds exactly past + n rows, rounded up to 256, and the
     last 64-key tile ends at the allocation's end.  Waves whose queries
     are all past n must not copy a K tile beyond it (they once did, in
@@ -138,7 +154,7 @@ def test_prefill_long_past_and_c4_adjacent(past, n):
 
 
 @pytest.mark.parametrize("n,past", [(1, 0), (129, 0), (200, 77), (300, 1000), (1000, 31)])
-def test_prefill_32_query_kernel_matches(n, past, monkeypatch):
+def test_prefill_32_query_kernel_matches(n, past, monkeypatch, grid):
     """The earlier 32-queries-per-wave kernel (MI_ATTN_PREFILL_QPW=32, read
     at each call) against the oracle, and against the default 64-query
     kernel on the same inputs."""
@@ -159,7 +175,7 @@ def test_prefill_32_query_kernel_matches(n, past, monkeypatch):
     assert_close(outs[0], outs[1], f"prefill qpw=32 vs 64 n={n} past={past}", atol=1e-3)
 
 
-def test_prefill_restart_after_late_large_scores():
+def test_prefill_restart_after_late_large_scores(form):
     """Key 300 scores ~20 (base 2) above the first tile's keys for every
     query of KV group 0 (each query has a component along r, the key is 28 r):
     with the 64-query kernel's reference max fixed at the first tile, that

@@ -28,7 +28,13 @@ def _filled(rng, past, capacity):
 
 
 @pytest.mark.parametrize("seed", range(16))
-def test_prefill_random_shapes(seed):
+@pytest.mark.parametrize("form", ["grid", "default"])
+def test_prefill_random_shapes(seed, form, monkeypatch):
+    """The prefill grid, and what a call of that size runs by default (short
+    prompts: one launch)."""
+    if form == "grid":
+        monkeypatch.setenv("MI_ATTN_DIRECT", "0")
+        monkeypatch.setenv("MI_ATTN_PREFILL_SPLIT", "0")
     rng = np.random.default_rng(1000 + seed)
     past = int(rng.integers(0, 1200))
     n = int(rng.integers(17, 260))
@@ -56,11 +62,14 @@ def test_verify_random_shapes(seed):
 
 
 @pytest.mark.parametrize("seed", range(8))
-def test_split_prefill_and_wide_verify_random_shapes(seed):
-    """Prefill after a past of 2048 rows or more (at most half of it new)
-    takes the split-K form, and verify of more than 4 tokens the wide form:
-    both run the prefill tiles over key chunks and merge the partials.
-    Random (past, n) with unaligned chunk ends, against the oracle."""
+def test_split_prefill_and_wide_verify_random_shapes(seed, monkeypatch):
+    """Prefill after a past of 2048 rows or more (at most half of it new) in
+    the split-K form, and verify of more than 4 tokens in the wide form (the
+    one-launch form and the token groups off): both run the prefill tiles over
+    key chunks and merge the partials.  Random (past, n) with unaligned chunk
+    ends, against the oracle."""
+    monkeypatch.setenv("MI_ATTN_DIRECT", "0")
+    monkeypatch.setenv("MI_ATTN_VERIFY_GROUPS", "0")
     rng = np.random.default_rng(3000 + seed)
     past = int(rng.integers(2048, 6000))
     n = int(rng.integers(5, 100))
