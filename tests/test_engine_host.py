@@ -92,3 +92,17 @@ def test_no_interrupt_runs_every_layer_and_advances(method, calls):
     assert eng.engine_pos() == 10 + n
     if method == "forward_batched":  # n = 20 > the verify limit: the prefill kernel
         assert {c[0] for c in calls} == {"attn_prefill"}
+
+
+def test_stream_handle_with_and_without_the_raw_call(monkeypatch):
+    A = E.attention
+    monkeypatch.setattr(A, "_device", lambda: 3)
+    monkeypatch.setattr(A, "_raw_stream", lambda device: 100 + device)
+    assert A._stream() == 103
+
+    class Stream:
+        cuda_stream = 55
+
+    monkeypatch.setattr(A, "_raw_stream", None)
+    monkeypatch.setattr(A.torch.cuda, "current_stream", lambda: Stream)
+    assert A._stream() == 55
