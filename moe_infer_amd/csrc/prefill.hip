@@ -664,16 +664,16 @@ extern "C" mi_status mi_attn_prefill(mi_kv* kv, int32_t layer, const mi_f16* q,
   // A few tokens after a long past: the prefill grid (one workgroup per 128
   // queries and head) would leave most CUs idle while each of its
   // workgroups walks the whole past; the split-K form of the same tiles
-  // spreads the past over the CUs, then merges.  Not while a graph is being
-  // captured unless the workspace already suffices (growing it is refused
-  // then).
+  // spreads the past over the CUs, then merges.  The grid needs no workspace:
+  // it runs where there is none to be had (no memory, or a graph being
+  // captured, under which it does not grow).
   if (prefill_split_k(past_pos, n)) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    MI_HIP(hipStreamIsCapturing(s, &cs));
-    if (cs == hipStreamCaptureStatusNone ||
-        kv->ws_bytes >= mi::wide_workspace_bytes(kv->G, past_pos, n))
+    void* ws;
+    if (mi::kv_workspace(kv, mi::wide_workspace_bytes(kv->G, past_pos, n), s, &ws) == MI_OK)
       return mi::attend_wide(kv, layer, (const _Float16*)q, (const _Float16*)gate,
                              (_Float16*)out, past_pos, n, s);
+    mi::clear_error();
+    (void)hipGetLastError();
   }
   PrefillArgs a;
   a.q = (const _Float16*)q;

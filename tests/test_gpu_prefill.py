@@ -230,6 +230,40 @@ def test_prefill_split_k_form(past, n, monkeypatch):
     assert_close(out, whole, f"split-K vs unsplit past={past} n={n}", atol=1e-3)
 
 
+def test_prefill_in_a_graph_without_a_workspace(monkeypatch):
+    """700 tokens after 1500 rows run split over the past, which takes a
+    workspace; captured on a handle that has none, the call records the prefill
+    grid instead of being refused.  Three replays, with eager work between,
+    against the eager grid, bit for bit."""
+    import torch
+    announce("prefill captured without a workspace")
+    past, n = 1500, 700
+    rng = np.random.default_rng(past)
+    k, v = f16(rng, past + n, G * D), f16(rng, past + n, G * D)
+    q, g = dev(f16(rng, n, H, D)), dev(f16(rng, n, H, D))
+    kn, vn = dev(k[past:]), dev(v[past:])
+    c = Cache(num_layers=1, capacity=past + n)
+    c.upload(0, k[:past], v[:past])
+    out = torch.empty_like(q)
+    monkeypatch.setenv("MI_ATTN_PREFILL_SPLIT", "0")
+    ref = attn_prefill(c, 0, q, kn, vn, past, gate=g).clone()  # the grid: no workspace
+    monkeypatch.delenv("MI_ATTN_PREFILL_SPLIT")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        attn_prefill(c, 0, q, kn, vn, past, gate=g, out=out)
+    other = Cache(num_layers=1, capacity=256)
+    other.upload(0, k[:200], v[:200])
+    for r in range(3):
+        out.fill_(7.0)
+        graph.replay()
+        attn_decode(other, 0, q[0], 200)
+        torch.cuda.synchronize()
+        assert torch.equal(ref.view(torch.int16), out.view(torch.int16)), f"replay {r}"
+    eager = attn_prefill(c, 0, q, kn, vn, past, gate=g)  # split, now that it may grow
+    assert_close(eager, host(ref), "split-K against the captured grid", atol=1e-3)
+
+
 def test_prefill_split_k_restart():
     """Scores of odd 64-key tiles far above even ones for some rows: chunks
     whose first tile is even take the restart path in the split-K form."""
