@@ -83,8 +83,8 @@ MI_HD inline PrefillWave64 prefill_wave64(int past, int n, int qtile, int qb, in
 // [kbeg, kbeg + chunk) of [0, past + n), positions relative to kbeg; its
 // row block holds tokens tok0 .. tok0 + 15, rows 64 qb .. + 63 being tokens
 // tok0 + 8 qb .. + 7 (each with the group's eight heads), token i seeing
-// keys up to past + i.  A chunk past every key its tokens see keeps one
-// tile, fully masked (empty partials).
+// keys up to past + i.  Only chunks that hold keys of the block are launched
+// (wide_place).
 MI_HD inline PrefillWave64 verify_wave64(int64_t past, int n, int64_t kbeg, int64_t chunk,
                                          int tok0, int qb, int kp) {
   PrefillWave64 p;
@@ -93,7 +93,6 @@ MI_HD inline PrefillWave64 verify_wave64(int64_t past, int n, int64_t kbeg, int6
   const int tend = n < tok0 + 16 ? n : tok0 + 16;  // the block's tokens
   int64_t end = past + tend - kbeg;                 // keys they see in the chunk
   if (end > chunk) end = chunk;
-  if (end < 1) end = 1;
   p.kv_len = (int)end;
   p.nt = (p.kv_len + kPrefillBK - 1) / kPrefillBK;
   p.koff = 32 * kp;
@@ -329,8 +328,8 @@ struct SplitPlan {
 // chunk of two heads moves 256 KiB and leaves one 8 KiB partial per head and
 // query token), at least one 32-key tile, at most 2048 keys (ragged batches
 // balance better with more workgroups), and at most kMaxSplitChunks chunks.
-// Chunks are whole 32-key tiles; the waves of a workgroup take its tiles
-// round-robin.  Decode rounds chunks to 32 keys: rounding up to 32 * NWH
+// Chunks are whole 32-key tiles; each wave of a workgroup takes a contiguous run
+// of its tiles.  Decode rounds chunks to 32 keys: rounding up to 32 * NWH
 // would leave up to half the CUs idle just above a power of two (ctx 32769:
 // 129 workgroups instead of 256, 21.0 against 18.1 us per call).  The
 // 32-column verify (nq > 2) keeps whole wave rounds (measured ~1 us faster

@@ -62,9 +62,10 @@ struct PrefillArgs {
   float scale_log2e;
 };
 
-// Wide verify (attn_verify_wide_kernel): workgroup = (key chunk, KV head);
-// rows are (token, query head of the group) pairs, row = 8 token + head;
-// keys [c chunk, (c + 1) chunk) of [0, past + n); unnormalised partials
+// Wide verify (attn_verify_wide_kernel): workgroup = (row block of 16 tokens,
+// key chunk that its tokens see, KV head), placed by mi::wide_place; rows are
+// (token, query head of the group) pairs, row = 8 token + head; keys [c chunk,
+// (c + 1) chunk) of [0, past + n); unnormalised partials
 // (O, m, l) go to part_o [G][nslots][ncols][D] / part_ml [..][2] for the
 // combine kernel (ncols = 8 n).
 struct VerifyArgs {

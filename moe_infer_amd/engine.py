@@ -11,9 +11,8 @@ per-layer q / k / v / gate projections and get the gated attention output.
                              then pos += 1 (fused_exp2.rs:989-1039)
   forward_batched(layers)    n tokens per layer, causal (batched.rs:129-312);
                              pos += n (fused_exp3.rs:291).  n <= VERIFY_MAX_TOKENS
-                             runs the split-K verify kernel (HBM-bound, the
-                             whole cache in one pass per 4 tokens), larger n
-                             the MFMA prefill kernel
+                             runs the verify call, larger n the prefill call
+                             (VERIFY_MAX_TOKENS below)
   forward_proj(layers) /     the same two steps from the f32 projections:
   forward_batched_proj(...)  per-head Q/K RMS norm + NeoX partial RoPE fused in
                              (cpu.rs:122-145, fused_exp2.rs:630-733)
@@ -89,9 +88,9 @@ class EngineSnapshot:
     mtp_pos: int
 
 
-# Largest token count forward_batched sends to mi_attn_verify (the decode
-# kernel's forms, above 20480 rows and 4 tokens the prefill tiles' split-K
-# form), the speculative-verify case; more tokens go to mi_attn_prefill, which
+# Largest token count forward_batched sends to mi_attn_verify (the speculative
+# verify: the decode kernel's forms, for more than 4 tokens above 20480 rows the
+# prefill tiles split over the past); more tokens go to mi_attn_prefill, which
 # itself runs short prompts in one launch and splits over the past when the
 # past is long next to them.
 VERIFY_MAX_TOKENS = 16
