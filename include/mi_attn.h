@@ -180,11 +180,14 @@ mi_status mi_attn_step(mi_kv* kv, int32_t layer, const mi_f16* q,
  * shaders.metal:2656-2792): append n rows k, v [n][G*D] at past_pos, then
  * query i (q [n][H][D]) attends rows [0, past_pos + i] inclusive; gate
  * [n][H][D] or NULL; out [n][H][D].  Short prompts (n (past + n/2) up to
- * 480000, 3200 rows) run in one launch; up to 1024 new tokens after a past of
+ * 480000, 3200 rows) run in one launch, but for those of more than about 128
+ * tokens after 2048 rows or more; up to 1024 new tokens after a past of
  * at least n rows (n/2 for up to 640) the split-K form of the MFMA
  * flash-attention kernel over key chunks plus a merge, which needs the
- * handle's workspace (grown on demand; under graph capture only when it already
- * suffices, else the unsplit kernel runs); anything else the unsplit kernel.
+ * handle's workspace (grown on demand; where it cannot grow, as under graph
+ * capture, the unsplit kernel runs); anything else the unsplit kernel.  These
+ * lines are those of one or two KV heads; with more, the unsplit kernel serves
+ * more of the sizes (the rules are in csrc/plan.h).
  * MI_ATTN_PREFILL_SPLIT=0 turns the split-K form off.
  * k = v = NULL: rows [past_pos, past_pos+n) are already in the cache (written
  * by mi_qk_norm_rope_append or mi_kv_append; len(layer) >= past_pos + n), no
@@ -201,7 +204,8 @@ mi_status mi_attn_prefill(mi_kv* kv, int32_t layer, const mi_f16* q,
  * the prefill's MFMA tiles over key chunks that reads each K/V tile once per 16
  * tokens (MI_ATTN_VERIFY_WIDE=0 runs one launch pair per four tokens instead),
  * then a merge; short contexts (1024 + 80 (n - 1) rows for up to 4 tokens, 1400
- * + 21 n for up to 16) in one launch.  Rollback afterwards is
+ * + 21 n for up to 16) in one launch.  More than two KV heads run the one pass
+ * from shorter contexts on (csrc/plan.h).  Rollback afterwards is
  * mi_kv_set_pos.  k = v = NULL as for mi_attn_prefill. */
 mi_status mi_attn_verify(mi_kv* kv, int32_t layer, const mi_f16* q,
                          const mi_f16* k, const mi_f16* v, const mi_f16* gate,

@@ -1743,11 +1743,11 @@ struct Span {
   const void* p;
   size_t bytes;
 };
-bool takes_direct(int64_t past, int32_t n, int H, const _Float16* gate, const _Float16* out,
-                  std::initializer_list<Span> inputs) {
-  if (!mi::direct_rows(past, n)) return false;
+bool takes_direct(const mi_kv* kv, int64_t past, int32_t n, const _Float16* gate,
+                  const _Float16* out, std::initializer_list<Span> inputs, bool prefill = false) {
+  if (!mi::direct_rows(kv->G, past, n, prefill)) return false;
   if (((uintptr_t)gate | (uintptr_t)out) & 7) return false;  // 8-byte accesses here only
-  const uintptr_t o0 = (uintptr_t)out, o1 = o0 + (size_t)n * H * D * sizeof(_Float16);
+  const uintptr_t o0 = (uintptr_t)out, o1 = o0 + (size_t)n * kv->H * D * sizeof(_Float16);
   for (const Span& s : inputs)
     if (s.p && (uintptr_t)s.p < o1 && o0 < (uintptr_t)s.p + s.bytes) return false;
   if (split_knobs().chunk > 0 || split_knobs().gh != 1 || split_knobs().wgs != 256) return false;
@@ -1822,12 +1822,12 @@ mi_status cache_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float
   // tokens after 2900 rows 33.9 us against 39.7, after 2100 36.5 against 33.0)
   const bool direct =
       (n <= 4 || wide) && (past_pos < 2400 || direct_slices(kv->G, n) > 1) &&
-      takes_direct(past_pos, n, kv->H, gate, out,
+      takes_direct(kv, past_pos, n, gate, out,
                    {{q, (size_t)n * kv->H * D * sizeof(_Float16)}, {k_new, rows_bytes},
                     {v_new, rows_bytes}});
   if (wide) {
     const bool groups =
-        !direct && mi::verify_groups(past_pos, n) && switched_on("MI_ATTN_VERIFY_GROUPS");
+        !direct && mi::verify_groups(kv->G, past_pos, n) && switched_on("MI_ATTN_VERIFY_GROUPS");
     if (!direct && !groups)
       return wide_attend(kv, layer, q, gate, out, past_pos, n, stream, k_new, v_new);
     // (the wide form's workspace too: a later captured call may count on what
@@ -1933,7 +1933,7 @@ mi_status attend_cache(mi_kv* kv, int32_t layer, const _Float16* q, const _Float
 
 bool attend_direct(mi_kv* kv, int32_t layer, const _Float16* q, const _Float16* gate,
                    _Float16* out, int64_t past, int32_t n, hipStream_t stream, mi_status* st) {
-  if (!takes_direct(past, n, kv->H, gate, out, {{q, (size_t)n * kv->H * D * sizeof(_Float16)}}))
+  if (!takes_direct(kv, past, n, gate, out, {{q, (size_t)n * kv->H * D * sizeof(_Float16)}}, true))
     return false;
   // Long pasts next to n: the split-K form serves them as well.  In one slice of
   // V, where the precision of its weights would have to be paid for (TILE), it is
@@ -2081,7 +2081,7 @@ extern "C" mi_status mi_attn_step_proj(mi_kv* kv, int32_t layer, const float* q_
   MI_TRY(mi::kv_workspace(kv, attend_workspace_bytes(kv->G, plan.max_chunks, 1), (hipStream_t)stream, &ws));
   const size_t q_bytes = (size_t)kv->H * 2 * D * sizeof(float);
   const size_t kv_bytes = (size_t)kv->G * D * sizeof(float), w_bytes = D * sizeof(uint16_t);
-  if (takes_direct(pos, 1, kv->H, nullptr, (const _Float16*)out,
+  if (takes_direct(kv, pos, 1, nullptr, (const _Float16*)out,
                    {{q_proj, q_bytes},
                     {k, kv_bytes},
                     {v, kv_bytes},

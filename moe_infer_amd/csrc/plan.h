@@ -277,15 +277,26 @@ inline WidePlan wide_plan(int G, int64_t past, int n) {
 // 1500 15.1 / 16.8, at 2000 19.3 / 16.9; 16 at 1500 15.1 / 18.0, at 2000 19.5 /
 // 18.2.
 // More tokens, without their append (against the prefill grid / the split-K
-// pass): 64 after 1000 rows 10.4 / 35.3 / 24.2, 128 after 3000 27.8 / 82.2 /
-// 28.9, 400 after 1000 30.3 / 45.1 / 32.8, 777 from none 25.5 / 30.9 / 42.3;
+// pass), two KV heads: 64 after 1000 rows 10.4 / 35.3 / 24.2, 128 after 3000 27.8 /
+// 82.2 / 28.9, 400 after 1000 30.3 / 45.1 / 32.8, 777 from none 25.5 / 30.9 / 42.3;
 // past the line: 300 after 1500 35.3 / 53.6 / 31.5, 1024 from none 36.6 / 37.0
 // / 36.6, 17 after 5000 33.6 / 119.7 / 25.0.
-inline bool direct_rows(int64_t past, int32_t n) {
-  const int64_t rows = past + n;
+// A prompt's line falls with the square of the KV heads: each adds its own
+// workgroups here, while those it adds to the grid find idle CUs (one launch
+// against the better of grid and split-K): 3 heads, 606 from none 31.1 / 33.1, 685
+// 32.8 / 32.5; 4 heads, 387 from none 24.4 / 26.0, 558 33.3 / 31.6, 959 after 20 61.2
+// / 42.9; 6 heads, 257 from none 21.1 / 23.4, 318 29.0 / 27.2; 8 heads, 200 from none
+// 20.4 / 21.7, 277 30.6 / 27.9, 876 94.9 / 57.9.  The alternative of a verify is the
+// split-K pass, which they add to as well: 4 heads, 125 after 1303 26.4 / 34.3, 129
+// after 1610 41.8 / 39.3; 8 heads, 203 after 1221 61.0 / 46.5; and where a workgroup
+// walks far: 8 heads, 59 after 966 22.7 / 33.1, 25 after 3017 44.2 / 38.6.
+inline bool direct_rows(int G, int64_t past, int32_t n, bool prefill) {
+  const int64_t rows = past + n, keys = n * (past + n / 2);
   if (n <= 4) return rows <= 1024 + 80 * (n - 1);
   if (n <= 16) return rows <= 1400 + 21 * n;
-  return rows <= 3200 && n * (past + n / 2) <= 480000;
+  if (rows > 3200 || keys > 480000) return false;
+  return prefill ? keys * G * G <= 2200000 && n * G <= 2080 - 60 * G
+                 : keys * G <= (G <= 2 ? 960000 : 860000) && rows * G <= 18000;
 }
 
 // Whether a verify of 5 to 16 tokens outside that runs as groups of four tokens
@@ -296,7 +307,19 @@ inline bool direct_rows(int64_t past, int32_t n) {
 // groups / wide): 8 tokens after 2300 rows 16.1 / 20.7, after 9001 18.8 / 26.0,
 // after 24000 27.6 / 28.2; 12 after 9001 19.8 / 30.9; 9 after 24000 31.0 / 29.7;
 // 16 after 16000 26.0 / 33.4, after 32000 40.2 / 38.1, after 65536 100 / 49.
-inline bool verify_groups(int64_t past, int32_t n) { return n <= 16 && past + n <= 20480; }
+// More heads leave fewer chunks to a group, and where a head's chunks do not fall
+// on the XCDs in turn, or three groups do not, L2 serves less of the rereads: 3
+// heads, 11 after 12177 rows 26.8 / 33.4, 13 after 13436 39.9 / 33.6; 4 heads, 11
+// after 16723 35.1 / 37.3 (given up for 10 after 10727, 32.1 / 29.9); 6 heads, 16
+// after 4907 32.5 / 37.1, 15 after 5740 42.5 / 37.1, 8 after 8846 28.3 / 34.1, 6 after
+// 12924 38.4 / 35.0; 8 heads, 9 after 6126 33.6 / 39.9, 10 after 7870 39.5 / 37.8, 16
+// after 7465 45.1 / 49.9 (given up for 13 after 6228, 44.3 / 41.1), after 12960 57.5 /
+// 49.9.
+inline bool verify_groups(int G, int64_t past, int32_t n) {
+  const int64_t rows = past + n, ng = (n + 3) / 4;
+  return n <= 16 && rows <= 20480 &&
+         rows * G * ng <= (8 % G ? 110000 : ng == 3 ? 163840 : 196608);
+}
 
 // Whether a prefill outside that takes the split-K pass and its merge rather
 // than the prefill grid (one workgroup per 128 queries and head): the grid is
@@ -307,9 +330,17 @@ inline bool verify_groups(int64_t past, int32_t n) { return n <= 16 && past + n 
 // after 16384 139 / 377.  Nowhere in 300 sizes of 100 to 1024 tokens did the
 // grid win; below the line the lead shrinks with the past (777 after 291 34.4 /
 // 38.1, 1024 from none 33.9 / 35.6), and with more tokens no CU is idle (1200
-// from none 39.2 / 39.1).
-inline bool prefill_split_rows(int64_t past, int32_t n) {
-  return n <= 1024 && past >= (n <= 640 ? n / 2 : n);
+// from none 39.2 / 39.1).  That is for up to two KV heads; with more the grid has
+// more workgroups and wins up to longer pasts: 4 heads, 630 after 993 62.6 / 58.4,
+// 432 after 362 39.9 / 37.3; 6 heads, 360 after 1036 56.3 / 51.0; 8 heads, 175 after
+// 263 38.6 / 32.7, 179 after 628 43.8 / 40.7; split-K takes 0.95 of the grid's time at
+// 477 after 980 (4 heads), 0.78 at 188 after 1356 (6), 0.97 at 190 after 1059 (8), and
+// loses where only some blocks get a second chunk (8 heads, 302 after 1482 75.2 /
+// 64.3).
+inline bool prefill_split_rows(int G, int64_t past, int32_t n) {
+  if (n > 1024) return false;
+  if (G <= 2) return past >= (n <= 640 ? n / 2 : n);
+  return past >= (int64_t)n * G / 2 && past >= 125 * G && (n * G <= 2048 || past >= 2048);
 }
 
 struct SplitKnobs {

@@ -584,10 +584,10 @@ mi_status launch_verify_wide(const PrefillArgs& a, const VerifyArgs& v, int grid
 // Whether mi_attn_prefill takes the split-K form (the wide verify's pass and
 // merge; mi::prefill_split_rows).  MI_ATTN_PREFILL_SPLIT=0 (read at each call)
 // turns it off.
-bool prefill_split_k(int64_t past, int32_t n) {
+bool prefill_split_k(int G, int64_t past, int32_t n) {
   const char* e = getenv("MI_ATTN_PREFILL_SPLIT");
   if (e && *e && atoi(e) == 0) return false;
-  return mi::prefill_split_rows(past, n);
+  return mi::prefill_split_rows(G, past, n);
 }
 
 // Queries per wave of the prefill kernel: 64 (attn_prefill64_kernel, the
@@ -668,7 +668,7 @@ extern "C" mi_status mi_attn_prefill(mi_kv* kv, int32_t layer, const mi_f16* q,
   // spreads the past over the CUs, then merges.  The grid needs no workspace:
   // it runs where there is none to be had (no memory, or a graph being
   // captured, under which it does not grow).
-  if (prefill_split_k(past_pos, n)) {
+  if (prefill_split_k(kv->G, past_pos, n)) {
     void* ws;
     if (mi::kv_workspace(kv, mi::wide_workspace_bytes(kv->G, past_pos, n), s, &ws) == MI_OK)
       return mi::attend_wide(kv, layer, (const _Float16*)q, (const _Float16*)gate,

@@ -227,7 +227,7 @@ int main() {
   // verify by token groups: the chunks cover the rows, a grid of one round of
   // workgroups where one chunk each would be
   long long cg = 0, bg = 0;
-  for (int G : {1, 2, 3, 4, 8})
+  for (int G : {1, 2, 3, 4, 6, 8})
     for (int ng = 2; ng <= 4; ng++)
       for (long long rows = 1; rows <= 20480; rows += (rows < 600 ? 1 : 13)) {
         const mi::SplitPlan p = mi::plan_groups(rows, ng, G, mi::SplitKnobs{1, 256, 0});
@@ -237,6 +237,40 @@ int main() {
         cg++;
       }
   std::printf("groups %lld %lld\n", cg, bg);
+
+  // Which form a call runs, at sizes where the forms differ by 4 % or more
+  // (the times are at the rules): D one launch, S split over the past, G the
+  // prefill grid, for prompts; D, T token groups, W the wide pass, for a verify.
+  struct Route {
+    bool prefill;
+    int G, past, n;
+    char form;
+  };
+  const Route routes[] = {
+      {true, 2, 0, 777, 'D'},     {true, 2, 1000, 400, 'D'},   {true, 2, 1500, 300, 'S'},
+      {true, 2, 1024, 512, 'S'},  {true, 3, 0, 606, 'D'},      {true, 4, 0, 387, 'D'},
+      {true, 4, 20, 959, 'G'},    {true, 4, 0, 558, 'G'},      {true, 4, 993, 630, 'G'},
+      {true, 4, 980, 477, 'S'},   {true, 6, 0, 257, 'D'},      {true, 6, 0, 318, 'G'},
+      {true, 6, 1036, 360, 'G'},  {true, 6, 1356, 188, 'S'},   {true, 8, 0, 200, 'D'},
+      {true, 8, 0, 277, 'G'},     {true, 8, 0, 876, 'G'},      {true, 8, 263, 175, 'G'},
+      {true, 8, 628, 179, 'G'},   {true, 8, 2107, 193, 'S'},   {false, 2, 9001, 12, 'T'},
+      {false, 2, 20400, 16, 'T'}, {false, 1, 20400, 16, 'T'},  {false, 2, 24000, 12, 'W'},
+      {false, 3, 12177, 11, 'T'}, {false, 3, 13436, 13, 'W'},  {false, 4, 16723, 6, 'T'},
+      {false, 4, 18196, 11, 'W'}, {false, 6, 5740, 15, 'W'},   {false, 6, 8846, 8, 'T'},
+      {false, 6, 12924, 6, 'W'},  {false, 8, 6126, 9, 'T'},    {false, 8, 7870, 10, 'W'},
+      {false, 8, 12960, 16, 'W'}, {false, 4, 1303, 125, 'D'},  {false, 8, 1221, 203, 'W'}, {false, 4, 1610, 129, 'W'},
+      {false, 8, 3017, 25, 'W'},  {false, 8, 966, 59, 'D'},    {false, 8, 6228, 13, 'W'},
+      {true, 8, 1482, 302, 'G'}};
+  long long cr = 0, br = 0;
+  for (const Route& r : routes) {
+    const char form = mi::direct_rows(r.G, r.past, r.n, r.prefill) ? 'D'
+                      : r.prefill ? (mi::prefill_split_rows(r.G, r.past, r.n) ? 'S' : 'G')
+                                  : (mi::verify_groups(r.G, r.past, r.n) ? 'T' : 'W');
+    br += form != r.form;
+    cr++;
+    if (form != r.form) std::fprintf(stderr, "G=%d past=%d n=%d: %c\n", r.G, r.past, r.n, form);
+  }
+  std::printf("routes %lld %lld\n", cr, br);
 
   long long cw = 0, bw = 0;
   for (long long past : {0LL, 1LL, 63LL, 64LL, 65LL, 700LL, 2048LL, 4096LL, 5000LL, 6500LL,

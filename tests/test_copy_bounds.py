@@ -72,3 +72,10 @@ def test_token_groups_run_in_one_round(model_output):
     workgroups than the 256 CUs take at once."""
     cases, bad = model_output["groups"]
     assert cases > 20000 and bad == 0
+
+
+def test_forms_by_size_and_heads(model_output):
+    """Each call runs the form that measured fastest at its size and number of
+    KV heads (41 sizes on both sides of the lines)."""
+    cases, bad = model_output["routes"]
+    assert cases == 41 and bad == 0
