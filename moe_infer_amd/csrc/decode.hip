@@ -1716,9 +1716,12 @@ mi_status wide_attend(mi_kv* kv, int32_t layer, const _Float16* q, const _Float1
   c.batch = 1;
   c.nslots = nchunks;
   // 16-byte lanes per column fill the CUs from 64 tokens on; for fewer with
-  // many chunks (16 tokens at 65536 rows: 114) a workgroup per column and
-  // 32-value slice does.  The rows form moves 8-byte pieces of gate and out.
-  if ((nchunks <= 16 || n >= 64) && !(((uintptr_t)gate | (uintptr_t)out) & 7))
+  // many chunks (16 tokens at 65536 rows: 114), or where a wave's walk over the
+  // chunks is long next to the columns (one KV head: 68 tokens in 49 chunks, 34.8
+  // us a call against 31.4; 120 in 32 36.8 against 40.7), a workgroup per column
+  // and 32-value slice does.  The rows form moves 8-byte pieces of gate and out.
+  if ((nchunks <= 16 || (n >= 64 && 8 * nchunks <= 5 * n * G)) &&
+      !(((uintptr_t)gate | (uintptr_t)out) & 7))
     MI_HIP(mi::launch("attn_combine", attn_combine_rows_kernel, dim3(n * 2, G), dim3(256), 0,
                       stream, c));
   else

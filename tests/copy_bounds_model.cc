@@ -94,7 +94,7 @@ static long long prefill64_violations(int past, int n, long long cap) {
 }
 
 // The wide verify / split-K prefill (attn_verify_wide_kernel): plan
-// mi::wide_plan (two KV heads); workgroup (row block rb of 16 tokens, chunk
+// mi::wide_plan (G KV heads); workgroup (row block rb of 16 tokens, chunk
 // c), placed by mi::wide_place as in the kernel: keys from kbeg = c * chunk,
 // wave (qb, kp) walking mi::verify_wave64's tiles with the 64-query kernel's copies (K(0) first; then K(min(t + 1,
 // nt - 1)) and V(t) at tile 0 and on active tiles, else K(t + 1) when
@@ -103,8 +103,8 @@ static long long prefill64_violations(int past, int n, long long cap) {
 // must be whole tiles, at most kMaxSplitChunks, and cover [0, past + n),
 // and each token's visible keys within a chunk must lie inside the tiles
 // its workgroup walks.
-static long long wide_violations(long long past, int n, long long cap) {
-  const mi::WidePlan wp = mi::wide_plan(2, past, n);
+static long long wide_violations(int G, long long past, int n, long long cap) {
+  const mi::WidePlan wp = mi::wide_plan(G, past, n);
   long long bad = 0;
   if (wp.chunk % mi::kPrefillBK || wp.nchunks > mi::kMaxSplitChunks ||
       (long long)wp.nchunks * wp.chunk < past + n)
@@ -112,15 +112,15 @@ static long long wide_violations(long long past, int n, long long cap) {
   // the workgroups name every (row block, chunk) with visible keys exactly once
   // per KV head
   const int nrb = (n + 15) / 16;
-  std::vector<char> named((size_t)nrb * wp.nchunks * 2, 0);
-  const mi::WideDeal deal = mi::wide_deal(2, past, n, wp.chunk, wp.nchunks);
+  std::vector<char> named((size_t)nrb * wp.nchunks * G, 0);
+  const mi::WideDeal deal = mi::wide_deal(G, past, n, wp.chunk, wp.nchunks);
   // one round of the 256 CUs, where the row blocks alone do not exceed it
-  if (nrb * 2 <= 256 && deal.grid > 256) bad++;
+  if (nrb * G <= 256 && deal.grid > 256) bad++;
   for (int i = 0; i < deal.grid; i++) {
       int rb, c, kvh;
-      if (!mi::wide_place(deal, 2, (int)past, n, (int)wp.chunk, i, rb, c, kvh)) continue;
-      if (rb < 0 || rb >= nrb || c < 0 || c >= wp.nchunks || kvh < 0 || kvh > 1 ||
-          named[((size_t)rb * wp.nchunks + c) * 2 + kvh]++) {
+      if (!mi::wide_place(deal, G, (int)past, n, (int)wp.chunk, i, rb, c, kvh)) continue;
+      if (rb < 0 || rb >= nrb || c < 0 || c >= wp.nchunks || kvh < 0 || kvh >= G ||
+          named[((size_t)rb * wp.nchunks + c) * G + kvh]++) {
         bad++;
         continue;
       }
@@ -154,8 +154,8 @@ static long long wide_violations(long long past, int n, long long cap) {
   }
   for (int rb = 0; rb < nrb; rb++)
     for (int c = 0; c < wp.nchunks; c++)
-      for (int kvh = 0; kvh < 2; kvh++)
-        if (named[((size_t)rb * wp.nchunks + c) * 2 + kvh] !=
+      for (int kvh = 0; kvh < G; kvh++)
+        if (named[((size_t)rb * wp.nchunks + c) * G + kvh] !=
             ((long long)c * wp.chunk < mi::wide_end((int)past, n, rb)))
           bad++;
   return bad;
@@ -273,13 +273,14 @@ int main() {
   std::printf("routes %lld %lld\n", cr, br);
 
   long long cw = 0, bw = 0;
-  for (long long past : {0LL, 1LL, 63LL, 64LL, 65LL, 700LL, 2048LL, 4096LL, 5000LL, 6500LL,
-                         12287LL, 12288LL, 20000LL, 65536LL,
-                         131071LL})
-    for (int n = 1; n <= 1100; n += (n < 40 ? 1 : 37)) {
-      bw += wide_violations(past, n, round_cap(past + n));
-      cw++;
-    }
+  for (int G : {1, 2, 3, 4, 6, 8})
+    for (long long past : {0LL, 1LL, 63LL, 64LL, 65LL, 700LL, 2048LL, 4096LL, 5000LL, 6500LL,
+                           12287LL, 12288LL, 20000LL, 65536LL,
+                           131071LL})
+      for (int n = 1; n <= 1100; n += (n < 40 ? 1 : 37)) {
+        bw += wide_violations(G, past, n, round_cap(past + n));
+        cw++;
+      }
   std::printf("wide %lld %lld\n", cw, bw);
   return 0;
 }
