@@ -54,10 +54,12 @@ struct RopeArgs {
 constexpr int kChunkPitch = 16 * 8 + 8;  // halves
 constexpr int kStageHalves = 32 * kChunkPitch;
 
-// Tokens from which K goes through LDS by block; fewer go row by row, a wave
-// each, which has the shorter chain: the call takes 2.7 / 2.8 / 3.4 us for 12
-// / 64 / 128 tokens, by block 3.9 / 4.1 / 4.5.
-constexpr int kKRowTokens = 192;
+// K rows (tokens times KV heads) from which K goes through LDS by block; fewer go
+// row by row, a wave each, which has the shorter chain: by block takes 1.24 of the
+// time for 195 tokens of two heads, 1.13 for 321, 0.99 for 457, 0.93 for 796; one
+// head 1.22 for 434, 0.99 for 957; 4 heads 1.11 for 139, 0.96 for 232; 8 heads 1.15 for
+// 73, 0.97 for 116 (rotary_dim 64; 128 to 256 cross 10 to 40 % later).
+constexpr int kKRows = 900;
 
 // RMS norm of one head, lane l holding columns 4l .. 4l+3.
 __device__ __forceinline__ void head_norm(const float4& x, const ushort4& wb, float eps,
@@ -116,7 +118,7 @@ __device__ __forceinline__ void lane_angles(const RopeArgs& a, int tok, int lane
   }
 }
 
-// One K row by one wave, stored in place (a few rows: kKRowTokens).
+// One K row by one wave, stored in place (a few rows: kKRows).
 template <bool BIG>
 __device__ __forceinline__ void k_row(const RopeArgs& a, int item) {
   constexpr int D = mi::kHeadDim;
@@ -231,7 +233,7 @@ __global__ void __launch_bounds__(256) qk_norm_rope_kernel(const RopeArgs a) {
   const int wg = blockIdx.y * gridDim.x + blockIdx.x;
   if (wg < a.nkv) {
     if (wg >= a.nk) v_rows(a, wg - a.nk);
-    else if (a.n < kKRowTokens) k_row<BIG>(a, wg * 4 + wave);
+    else if (a.n * a.G < kKRows) k_row<BIG>(a, wg * 4 + wave);
     else k_rows(a, wg, lds);
     return;
   }
@@ -316,7 +318,7 @@ extern "C" mi_status mi_qk_norm_rope_append(mi_kv* kv, int32_t layer, const floa
   mi::rope_inv_freq(rope_theta, rotary_dim, a.inv_freq);
 
   const int64_t last = pos + n - 1;
-  const bool by_row = n < kKRowTokens;
+  const bool by_row = (int64_t)n * kv->G < kKRows;
   a.nk = by_row ? (n * kv->G + 3) / 4
                 : (int)(2 * (last / MI_KV_KBLOCK - pos / MI_KV_KBLOCK + 1) * kv->G);
   a.nkv = a.nk + (int)((last / MI_KV_VBLOCK - pos / MI_KV_VBLOCK + 1) * kv->G);

@@ -125,11 +125,15 @@ def test_rotary_dims(rot):
     run_case(777, 5, rot=rot)
 
 
-# K by row up to 191 tokens, by 16 rows of a cache block above; first and last
-# blocks partly covered, and two angles a lane from rotary_dim 136 on.
+# K by row up to 449 tokens (two KV heads), by 16 rows of a cache block above;
+# first and last blocks partly covered, and two angles a lane from rotary_dim 136
+# on.
 @pytest.mark.parametrize("pos,n,rot", [(5, 191, 64), (5, 192, 64), (13, 193, 64), (32, 224, 64),
                                        (28, 200, 0), (3, 203, 8), (7, 211, 128), (9, 197, 136),
-                                       (30, 195, 256), (2, 17, 136)])
+                                       (30, 195, 256), (2, 17, 136),
+                                       (5, 449, 64), (5, 450, 64), (13, 451, 64), (32, 480, 64),
+                                       (28, 460, 0), (3, 463, 8), (7, 471, 128), (9, 457, 136),
+                                       (30, 455, 256)])
 def test_block_and_row_forms(pos, n, rot):
     run_case(pos, n, rot=rot, prefill_rows=pos + n + 40, f32_slack=True)
 
