@@ -185,15 +185,17 @@ MI_HD inline void wide_item(int past, int n, int chunk, int idx, int& rb, int& c
 //              share its L2
 //   else       (item, KV head), the head fastest: the blocks of a chunk one
 //              after the other
-// Measured (us, by block / runs / by item, from HBM), two KV heads: 17 tokens after
+// What decides is the K and V of all heads that the blocks share, and whether by
+// block a chunk's blocks fall on one XCD (a pitch of whole rounds) as well.
+// Measured (us, by block / runs / by item, from HBM; two KV heads): 17 tokens after
 // 3500 rows 25.3 / 26.0 / 24.7, after 9000 25.3 / 27.8 / 26.6, after 20000 30.9 / 29.0
-// / 32.5; 40 after 4500 29.6 / 32.1 / 27.5, after 12000 31.9 / 31.8 / 33.6, after
-// 32000 44.7 / 44.4 / 49.4; 51 after 49354 83.6 / 72.8 / 85.5; 64 after 64000 82.2 /
-// 82.8 / 93.9; 128 after 8000 37.4 / 38.2 / 35.6, after 64000 136.3 / 136.2 / 139.2.
-// What decides is the K and V of all heads that the blocks share: over 2200 sizes
-// of 1 to 8 heads the lines below are on average 0.6 % off the best of the three
-// (with lines in rows 1.7 %): 1 head, 28 after 12832 29.0 / 31.3 / 28.5; 3 heads, 97
-// after 10056 47.9 / 48.4 / 53.9, 71 after 11540 51.4 / 45.2 / 50.7.
+// / 32.5, after 65000, where the pitch is whole rounds, 52.0 / 53.0 / -; 49 after
+// 12000 (whole rounds) 35.1 / 35.7 / 39.7; 51 after 49354 83.6 / 72.8 / 85.5; 128 after
+// 8000 37.4 / 38.2 / 35.6, after 64000 136.3 / 136.2 / 139.2; 1 head, 28 after 12832 29.0
+// / 31.3 / 28.5; 3 heads, 71 after 11540 51.4 / 45.2 / 50.7.  The lines below are where
+// the means of 1800 sizes of 1 to 8 heads cross: in whole rounds by block takes
+// 1.01 to 1.05 of by item below 18000 and 0.88 to 0.99 above; else by block is up to
+// 5 % ahead of the others from 8000 or 13000 on, runs above 13000 to 24000.
 // A single row block (a verify of up to 16 tokens) goes by block: its look-up is a
 // division, the others' would cost it 0.4 of 35 us.
 struct WideDeal {
@@ -212,18 +214,16 @@ inline WideDeal wide_deal(int G, int64_t past, int n, int64_t chunk, int nchunks
   d.grid = d.items * G;
   const int nrb = (n + 15) / 16;
   const int64_t kv = G * past;
-  // (2, 4 or 8 heads fall on the XCDs in turn: each of them reads one head's K/V)
+  const bool shared = nchunks * G % 8 == 0;  // by block, a chunk's blocks are on one XCD
+  const bool fits = nrb <= 8 && nrb * nchunks * G <= 256;
+  // (2, 4 and 8 heads fall on the XCDs in turn: each reads one head's K/V, and gains
+  // from runs later)
   const bool spread = G == 1 || 8 % G;
-  const bool runs = nrb > 1 && kv >= (nrb < 4   ? 32000 - 4000 * nrb
-                                      : nrb < 6 ? 18000
-                                      : spread  ? 12288
-                                                : 16000);
-  const bool by_block = nrb == 1 || (!runs && nrb <= (spread ? 8 : 4) &&
-                                     kv >= (nrb < 4 ? 13000 : 10000));
-  if (by_block && (nrb == 1 || nrb * nchunks * G <= 256)) {
+  const bool far = kv >= (nrb == 2 && !shared ? 24000 : nrb > 4 && spread ? 13000 : 18000);
+  if (nrb == 1 || (fits && (shared ? far : !far && kv >= (nrb < 4 ? 13000 : 8000)))) {
     d.pitch = nchunks * G;
     d.grid = nrb * d.pitch;
-  } else if (runs) {
+  } else if (far) {
     d.run = (d.grid + 7) / 8;
     d.grid = 8 * d.run;
   }
