@@ -10,7 +10,7 @@
 // rows of a V block.  Row by row, K left in 8-byte and V in 2-byte pieces of
 // lines that other CUs also wrote.  Measured per call against four sincosf and
 // row-wise stores: 4096 tokens 62.6 -> 36.4 us (6.2 TB/s), 1900 tokens 27.1 ->
-// 18.5, 333 tokens 7.4 -> 5.4, 12 tokens 3.6 -> 2.7.  Two, four or eight heads
+// 18.5, 333 tokens 7.4 -> 4.9 (by row), 12 tokens 3.6 -> 2.7.  Two, four or eight heads
 // to a wave (more loads in flight, fewer sincosf): 1900 tokens 18.4, 19.1 and
 // 21.1 us, 12 tokens 2.9, 3.3 and 4.4.
 //
